@@ -240,7 +240,8 @@ def prepare(case, seed):
     if op == "r2c":
         st["x"] = s["x"].to(dt)
     elif op == "c2r":
-        st["k"] = s["k"].to(torch.complex64 if dt == torch.float32 else torch.complex128)
+        # row-major, as PMesh.r2c returns it
+        st["k"] = s["k"].to(torch.complex64 if dt == torch.float32 else torch.complex128).contiguous()
     elif op == "paint":
         st["X"] = s["X"].to(dt)
     elif op == "paint_vjp":
