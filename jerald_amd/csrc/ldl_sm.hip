@@ -32,6 +32,7 @@
 // starmap^gamma3, W = exp(-k/kli - khi/k) k^nui + xi.
 #include "cic.h"
 #include "fft.h"
+#include "stencil.h"
 
 namespace ldl {
 
@@ -540,225 +541,6 @@ k_sm_x_bwd(ColGeom g, const c2<T>* Sq, const c2<T>* __restrict__ tw, const c2<T>
 #pragma unroll
         for (int j = 0; j < NP; j++) part[blockIdx.x * NP + j] = acc[j];
     }
-}
-
-// ------------------------------------------- real-space derivative stencils
-// The derivative symbol of k_axis_tables, D_d = (45 sin t - 9 sin 2t +
-// sin 3t) / (30 h_d) with t = 2 pi n / N_d, is that of the 6th-order central
-// difference
-//   diff_d(a)[x] = 45 (a[x+1] - a[x-1]) - 9 (a[x+2] - a[x-2]) + (a[x+3] - a[x-3])
-// along axis d (circular): a circular shift by s multiplies transform bin n
-// by exp(+-2 pi i n s / N), so the transform of diff_d(a) / (60 h_d) is
-// i D_d times the transform of a, and the inverse transform of -i D_d P is
-// -diff_d(phi) / (60 h_d) with phi the inverse transform of P.  The layer
-// therefore transforms one mesh each way: k_grad6 turns the potential phi
-// into the forces F_d = -diff_d(phi) / (60 h_d), and k_div6 turns the
-// painted gradient meshes g_d into sum_d diff_d(g_d) / (60 h_d), whose
-// transform is the sum_d i D_d of theirs.
-//
-// A workgroup of 4 st_tz<T>() threads covers kStTY (y) x st_tz<T>() (z) cells (each thread
-// 4 cells along y at one z) and marches through kStXC x planes: the x
-// difference comes from a 7-plane register queue per cell, the y and z
-// differences from the current plane staged in LDS with 3-cell halos.  All
-// indices are wrapped, so a tile larger than the mesh reads valid periodic
-// values and only its stores are bounded.
-constexpr int kStTY = 16, kStXC = 64;
-// z width of a tile: its 3-cell z halo costs two extra cache lines per row, so
-// wider rows fetch less (FP32, 512^3: grad6 0.500 -> 0.466 ms, div6 0.471 ->
-// 0.432 ms from 64 to 256); FP64 keeps 128 (at 1024 threads its divergence
-// would spill)
-template <typename T> constexpr int st_tz() { return sizeof(T) == 4 ? 256 : 128; }
-
-struct StGeom {
-    int n0, n1, n2, tiles_y, tiles_z, chunks;
-};
-
-__device__ __forceinline__ int st_wrap(int v, int n) { return ((v % n) + n) % n; }
-
-template <typename T>
-__device__ __forceinline__ T st_diff(T m3, T m2, T m1, T p1, T p2, T p3) {
-    return T(45) * (p1 - m1) - T(9) * (p2 - m2) + (p3 - m3);
-}
-
-template <int TZ> struct StTile {
-    int x0, x1, y0, z0, tz, yg;
-    int zw, yw[4];
-    bool zok, yok[4];
-    // halo cells this thread stages: y-halo rows hy[0..1] (row index of the
-    // (kStTY + 6)-row plane, -1 none) at its own z; one z-halo cell (zrow, zcol)
-    int hy[2], hyw[2], zrow, zcol, zyw, zzw;
-    __device__ __forceinline__ StTile(const StGeom& g) {
-        const int t = (int)xcd_tile(blockIdx.x, gridDim.x);
-        const int tzt = t % g.tiles_z, tyt = (t / g.tiles_z) % g.tiles_y, xc = t / (g.tiles_z * g.tiles_y);
-        x0 = xc * kStXC;
-        x1 = x0 + kStXC < g.n0 ? x0 + kStXC : g.n0;
-        y0 = tyt * kStTY;
-        z0 = tzt * TZ;
-        tz = threadIdx.x % TZ;
-        yg = threadIdx.x / TZ;
-        zw = st_wrap(z0 + tz, g.n2);
-        zok = z0 + tz < g.n2;
-#pragma unroll
-        for (int c = 0; c < 4; c++) {
-            const int y = y0 + 4 * yg + c;
-            yw[c] = st_wrap(y, g.n1);
-            yok[c] = y < g.n1;
-        }
-        // y halo: rows 0..2 and kStTY+3..kStTY+5; thread rows yg and yg + 4
-#pragma unroll
-        for (int h = 0; h < 2; h++) {
-            const int r = yg + 4 * h;
-            hy[h] = r < 6 ? (r < 3 ? r : kStTY + r) : -1;
-            hyw[h] = st_wrap(y0 + (hy[h] < 0 ? 0 : hy[h]) - 3, g.n1);
-        }
-        // z halo: kStTY rows x 6 columns (0..2, TZ+3..TZ+5), threads 0..95
-        const int tt = threadIdx.x;
-        zrow = tt < 6 * kStTY ? tt / 6 : -1;
-        const int k = tt - (tt / 6) * 6;
-        zcol = k < 3 ? k : TZ + k;
-        zyw = st_wrap(y0 + (zrow < 0 ? 0 : zrow), g.n1);
-        zzw = st_wrap(z0 + zcol - 3, g.n2);
-    }
-};
-
-// Forces F (N0, N1, N2, 3), interleaved per cell, from the potential phi.
-template <typename T>
-__global__ void __launch_bounds__(4 * st_tz<T>()) k_grad6(const T* __restrict__ phi, T* __restrict__ F, StGeom g, T cx, T cy, T cz) {
-    constexpr int TZ = st_tz<T>();
-    __shared__ T pl[kStTY + 6][TZ + 6];
-    const StTile<TZ> tl(g);
-    if (tl.x0 >= g.n0) return;  // uniform over the workgroup
-    const int64_t ps = (int64_t)g.n1 * g.n2;
-    auto at = [&](int x, int y, int z) { return phi[(int64_t)st_wrap(x, g.n0) * ps + (int64_t)y * g.n2 + z]; };
-    T q[4][7];
-#pragma unroll
-    for (int c = 0; c < 4; c++)
-#pragma unroll
-        for (int k = 0; k < 7; k++) q[c][k] = at(tl.x0 - 3 + k, tl.yw[c], tl.zw);
-    T hy0 = at(tl.x0, tl.hyw[0], tl.zw), hy1 = tl.hy[1] >= 0 ? at(tl.x0, tl.hyw[1], tl.zw) : T(0);
-    T hz = tl.zrow >= 0 ? at(tl.x0, tl.zyw, tl.zzw) : T(0);
-    for (int x = tl.x0; x < tl.x1; x++) {
-        __syncthreads();  // the previous plane's reads are done
-#pragma unroll
-        for (int c = 0; c < 4; c++) pl[4 * tl.yg + c + 3][tl.tz + 3] = q[c][3];
-        pl[tl.hy[0]][tl.tz + 3] = hy0;
-        if (tl.hy[1] >= 0) pl[tl.hy[1]][tl.tz + 3] = hy1;
-        if (tl.zrow >= 0) pl[tl.zrow + 3][tl.zcol] = hz;
-        __syncthreads();
-        // next plane's halo and the queue head, in flight during this plane
-        T head[4];
-        const bool more = x + 1 < tl.x1;
-        if (more) {
-#pragma unroll
-            for (int c = 0; c < 4; c++) head[c] = at(x + 4, tl.yw[c], tl.zw);
-            hy0 = at(x + 1, tl.hyw[0], tl.zw);
-            if (tl.hy[1] >= 0) hy1 = at(x + 1, tl.hyw[1], tl.zw);
-            if (tl.zrow >= 0) hz = at(x + 1, tl.zyw, tl.zzw);
-        }
-        if (tl.zok) {
-#pragma unroll
-            for (int c = 0; c < 4; c++) {
-                if (!tl.yok[c]) continue;
-                const int ly = 4 * tl.yg + c + 3, lz = tl.tz + 3;
-                const T dx = st_diff(q[c][0], q[c][1], q[c][2], q[c][4], q[c][5], q[c][6]);
-                const T dy = st_diff(pl[ly - 3][lz], pl[ly - 2][lz], pl[ly - 1][lz], pl[ly + 1][lz], pl[ly + 2][lz], pl[ly + 3][lz]);
-                const T dz = st_diff(pl[ly][lz - 3], pl[ly][lz - 2], pl[ly][lz - 1], pl[ly][lz + 1], pl[ly][lz + 2], pl[ly][lz + 3]);
-                T* o = F + 3 * ((int64_t)x * ps + (int64_t)(tl.y0 + 4 * tl.yg + c) * g.n2 + (tl.z0 + tl.tz));
-                o[0] = -cx * dx;
-                o[1] = -cy * dy;
-                o[2] = -cz * dz;
-            }
-        }
-        if (more) {
-#pragma unroll
-            for (int c = 0; c < 4; c++) {
-#pragma unroll
-                for (int k = 0; k < 6; k++) q[c][k] = q[c][k + 1];
-                q[c][6] = head[c];
-            }
-        }
-    }
-}
-
-// Divergence out = sum_d c_d diff_d(g_d) of the meshes g (3 consecutive
-// (N0, N1, N2) meshes) into a real mesh.
-template <typename T>
-__global__ void __launch_bounds__(4 * st_tz<T>()) k_div6(const T* __restrict__ gm, T* __restrict__ out, StGeom g, T cx, T cy, T cz) {
-    constexpr int TZ = st_tz<T>();
-    __shared__ T ly_[kStTY + 6][TZ];
-    __shared__ T lz_[kStTY][TZ + 6];
-    const StTile<TZ> tl(g);
-    if (tl.x0 >= g.n0) return;  // uniform over the workgroup
-    const int64_t ps = (int64_t)g.n1 * g.n2, cells = ps * g.n0;
-    const T* gx = gm;
-    const T* gy = gm + cells;
-    const T* gz = gm + 2 * cells;
-    auto at = [&](const T* a, int x, int y, int z) { return a[(int64_t)st_wrap(x, g.n0) * ps + (int64_t)y * g.n2 + z]; };
-    T q[4][7], vy[4], vz[4];
-#pragma unroll
-    for (int c = 0; c < 4; c++) {
-#pragma unroll
-        for (int k = 0; k < 7; k++) q[c][k] = at(gx, tl.x0 - 3 + k, tl.yw[c], tl.zw);
-        vy[c] = at(gy, tl.x0, tl.yw[c], tl.zw);
-        vz[c] = at(gz, tl.x0, tl.yw[c], tl.zw);
-    }
-    T hy0 = at(gy, tl.x0, tl.hyw[0], tl.zw), hy1 = tl.hy[1] >= 0 ? at(gy, tl.x0, tl.hyw[1], tl.zw) : T(0);
-    T hz = tl.zrow >= 0 ? at(gz, tl.x0, tl.zyw, tl.zzw) : T(0);
-    for (int x = tl.x0; x < tl.x1; x++) {
-        __syncthreads();  // the previous plane's reads are done
-#pragma unroll
-        for (int c = 0; c < 4; c++) {
-            ly_[4 * tl.yg + c + 3][tl.tz] = vy[c];
-            lz_[4 * tl.yg + c][tl.tz + 3] = vz[c];
-        }
-        ly_[tl.hy[0]][tl.tz] = hy0;
-        if (tl.hy[1] >= 0) ly_[tl.hy[1]][tl.tz] = hy1;
-        if (tl.zrow >= 0) lz_[tl.zrow][tl.zcol] = hz;
-        __syncthreads();
-        T head[4];
-        const bool more = x + 1 < tl.x1;
-        if (more) {
-#pragma unroll
-            for (int c = 0; c < 4; c++) {
-                head[c] = at(gx, x + 4, tl.yw[c], tl.zw);
-                vy[c] = at(gy, x + 1, tl.yw[c], tl.zw);
-                vz[c] = at(gz, x + 1, tl.yw[c], tl.zw);
-            }
-            hy0 = at(gy, x + 1, tl.hyw[0], tl.zw);
-            if (tl.hy[1] >= 0) hy1 = at(gy, x + 1, tl.hyw[1], tl.zw);
-            if (tl.zrow >= 0) hz = at(gz, x + 1, tl.zyw, tl.zzw);
-        }
-        if (tl.zok) {
-#pragma unroll
-            for (int c = 0; c < 4; c++) {
-                if (!tl.yok[c]) continue;
-                const int r = 4 * tl.yg + c, z = tl.tz;
-                const T dx = st_diff(q[c][0], q[c][1], q[c][2], q[c][4], q[c][5], q[c][6]);
-                const T dy = st_diff(ly_[r][z], ly_[r + 1][z], ly_[r + 2][z], ly_[r + 4][z], ly_[r + 5][z], ly_[r + 6][z]);
-                const T dz = st_diff(lz_[r][z], lz_[r][z + 1], lz_[r][z + 2], lz_[r][z + 4], lz_[r][z + 5], lz_[r][z + 6]);
-                out[(int64_t)x * ps + (int64_t)(tl.y0 + r) * g.n2 + (tl.z0 + z)] = cx * dx + cy * dy + cz * dz;
-            }
-        }
-        if (more) {
-#pragma unroll
-            for (int c = 0; c < 4; c++) {
-#pragma unroll
-                for (int k = 0; k < 6; k++) q[c][k] = q[c][k + 1];
-                q[c][6] = head[c];
-            }
-        }
-    }
-}
-
-template <typename T> static StGeom st_geom(const Mesh& m) {
-    StGeom g;
-    g.n0 = (int)m.n0;
-    g.n1 = (int)m.n1;
-    g.n2 = (int)m.n2;
-    g.tiles_y = (int)((m.n1 + kStTY - 1) / kStTY);
-    g.tiles_z = (int)((m.n2 + st_tz<T>() - 1) / st_tz<T>());
-    g.chunks = (int)((m.n0 + kStXC - 1) / kStXC);
-    return g;
 }
 
 // One axis of a separable Gaussian smoothing, W = exp(-|k|^2 sigma^2 / 2) =
@@ -1619,11 +1401,8 @@ static int sm_layer_fwd(int kind, const T* pos, const ldl_pos_desc* pdesc, int64
         if ((rc = colpass<T, +1>(m.n1, m.n0, nh, m.n1 * hp, hp, tw, PlainColOp<T>{P.spec3, P.spec3, T(1)}, st))) return rc;
         if ((rc = zpass_c2r<T>(nrows, m.n2, tw, HalfRowLoad<T>{P.spec3, hp}, RealRowStore<T>{phi, m.n2, T(1)}, st, nullptr)))
             return rc;
-        const StGeom sg = st_geom<T>(m);
-        KTimer _t("grad6", st);
-        hipLaunchKernelGGL(k_grad6<T>, dim3((unsigned)(sg.chunks * sg.tiles_y * sg.tiles_z)), dim3(4 * st_tz<T>()), 0, st, phi, F, sg,
-                           (T)((double)m.n0 / (60.0 * pdesc->box[0])), (T)((double)m.n1 / (60.0 * pdesc->box[1])),
-                           (T)((double)m.n2 / (60.0 * pdesc->box[2])));
+        launch_grad6<T>(m, phi, F, (T)((double)m.n0 / (60.0 * pdesc->box[0])), (T)((double)m.n1 / (60.0 * pdesc->box[1])),
+                        (T)((double)m.n2 / (60.0 * pdesc->box[2])), st);
     } else {
         if ((rc = colpass<T, +1>(m.n1, 3 * m.n0, nh, m.n1 * hp, hp, tw, PlainColOp<T>{P.spec3, P.spec3, T(1)}, st, "colpass3"))) return rc;
         if ((rc = zpass_c2r<T>(3 * nrows, m.n2, tw, Tri3RowLoad<T>{P.spec3, P.spec3 + hc, P.spec3 + 2 * hc, hp},
@@ -1681,13 +1460,8 @@ static int sm_layer_bwd(int kind, const T* pos, const ldl_pos_desc* pdesc, int64
     const bool p2 = fft_mesh_pow2(m);
     if (p2) {
         T* dv = reinterpret_cast<T*>(P.spec3 + 2 * hc);  // a real mesh in the free third spectrum
-        const StGeom sg = st_geom<T>(m);
-        {
-            KTimer _t("div6", st);
-            hipLaunchKernelGGL(k_div6<T>, dim3((unsigned)(sg.chunks * sg.tiles_y * sg.tiles_z)), dim3(4 * st_tz<T>()), 0, st, P.mesh3, dv, sg,
-                               (T)((double)m.n0 / (60.0 * pdesc->box[0])), (T)((double)m.n1 / (60.0 * pdesc->box[1])),
-                               (T)((double)m.n2 / (60.0 * pdesc->box[2])));
-        }
+        launch_div6<T>(m, P.mesh3, dv, (T)((double)m.n0 / (60.0 * pdesc->box[0])), (T)((double)m.n1 / (60.0 * pdesc->box[1])),
+                       (T)((double)m.n2 / (60.0 * pdesc->box[2])), st);
         if ((rc = zpass_r2c<T>(nrows, m.n2, tw, RealRowLoad<T>{dv, m.n2}, HalfRowStore<T>{P.spec3, hp, T(1)}, st))) return rc;
         if ((rc = colpass<T, -1>(m.n1, m.n0, nh, m.n1 * hp, hp, tw, PlainColOp<T>{P.spec3, P.spec3, T(1)}, st))) return rc;
     } else {
