@@ -647,8 +647,9 @@ k_x_realfilter(ColGeom g, const c2<T>* __restrict__ tw, c2<T>* __restrict__ io, 
 // iz >= nh are skipped), which do what the fused x kernels do between their
 // transforms.
 
-// out3[d] = -i D_d (cpot alpha G U [+ a G2 S2])
-template <typename T, bool HI>
+// PHI: out3 = P = cpot alpha G U [+ a G2 S2], the potential's spectrum; else
+// the three force spectra out3[d] = -i D_d P.
+template <typename T, bool HI, bool PHI>
 __global__ void __launch_bounds__(256) k_sm_filter_fwd(const c2<T>* __restrict__ U, c2<T>* __restrict__ out3, int64_t hcells, int64_t n1,
                                                        int64_t nh, int64_t hp, KTabs<T> kt, SmFilter<T> fl, T a1e2, Src2<T> s2) {
     for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < hcells; i += (int64_t)gridDim.x * blockDim.x) {
@@ -663,16 +664,20 @@ __global__ void __launch_bounds__(256) k_sm_filter_fwd(const c2<T>* __restrict__
             const T G2 = s2.a * s2.fl.G(k2);
             p = c2<T>{p.x + G2 * sv.x, p.y + G2 * sv.y};
         }
-        const T D[3] = {kt.D[0][ix], kt.D[1][iy], kt.D[2][iz]};
+        if constexpr (PHI) {
+            out3[i] = p;
+        } else {
+            const T D[3] = {kt.D[0][ix], kt.D[1][iy], kt.D[2][iz]};
 #pragma unroll
-        for (int d = 0; d < 3; d++) out3[d * hcells + i] = c2<T>{D[d] * p.y, -D[d] * p.x};
+            for (int d = 0; d < 3; d++) out3[d * hcells + i] = c2<T>{D[d] * p.y, -D[d] * p.x};
+        }
     }
 }
 
-// Q = sum_d i D_d S_d; FP64 partials (alpha, kh, kl, nu; HI also alpha2,
+// Q = S3 (PHI: the divergence's spectrum), else sum_d i D_d S_d; FP64 partials (alpha, kh, kl, nu; HI also alpha2,
 // kh2, kl2, nu2, gamma2) per workgroup into part[NP * block + j]; out =
 // cpot alpha G Q (out may alias S3's first spectrum).
-template <typename T, bool HI>
+template <typename T, bool HI, bool PHI>
 __global__ void __launch_bounds__(256) k_sm_filter_bwd(const c2<T>* S3, const c2<T>* __restrict__ U, c2<T>* out, int64_t hcells, int64_t n1,
                                                        int64_t nh, int64_t hp, int64_t n2, int64_t zdbl, KTabs<T> kt, SmFilter<T> fl, T a1e2, double gkh,
                                                        double gkl, double cpot, double alpha, int alpha_rule, Src2<T> s2,
@@ -683,12 +688,16 @@ __global__ void __launch_bounds__(256) k_sm_filter_bwd(const c2<T>* S3, const c2
     for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < hcells; i += (int64_t)gridDim.x * blockDim.x) {
         const int64_t iz = i % hp, iy = (i / hp) % n1, ix = i / (hp * n1);
         if (iz >= nh) continue;
-        const T D[3] = {kt.D[0][ix], kt.D[1][iy], kt.D[2][iz]};
         c2<T> q = c2<T>{T(0), T(0)};
+        if constexpr (PHI) {
+            q = S3[i];
+        } else {
+            const T D[3] = {kt.D[0][ix], kt.D[1][iy], kt.D[2][iz]};
 #pragma unroll
-        for (int d = 0; d < 3; d++) {
-            const c2<T> v = S3[d * hcells + i];
-            q = c2<T>{q.x - D[d] * v.y, q.y + D[d] * v.x};  // += i D v
+            for (int d = 0; d < 3; d++) {
+                const c2<T> v = S3[d * hcells + i];
+                q = c2<T>{q.x - D[d] * v.y, q.y + D[d] * v.x};  // += i D v
+            }
         }
         const T G = xbwd_cell<T, HI>(fl, s2, kt.knorm2(ix, iy, iz), q, U[i], i, xbwd_weights(iz, n2, zdbl, alpha_rule), cpot, apot, gkh,
                                      gkl, acc);
@@ -1324,6 +1333,15 @@ static int check_prm(const double* prm, int n) {
     return LDL_OK;
 }
 
+// Whether the layer transforms one mesh each way, the potential forward and the
+// divergence backward, with the derivatives taken in real space (k_grad6,
+// k_div6), or the three force and gradient spectra with the derivative symbol
+// applied in them.  One mesh is a third of the transform work (FP64 384^3
+// forward layer 9.05 -> 6.30 ms); FP32 meshes that are not powers of two keep
+// the symbol: differencing an FP32 potential rounds differently, which moves
+// their FP64-reduced gradients by up to 5e-8.
+template <typename T> inline bool layer_one_mesh(const Mesh& m) { return sizeof(T) == 8 || fft_mesh_pow2(m); }
+
 // Layer kinds: 0 sm, 1 dm, 2 HI (prm has 10 entries; star and S2buf used).
 enum { kKindSm = 0, kKindDm = 1, kKindHi = 2 };
 
@@ -1388,15 +1406,16 @@ static int sm_layer_fwd(int kind, const T* pos, const ldl_pos_desc* pdesc, int64
     } else {
         if ((rc = colpass<T, -1>(m.n0, m.n1, nh, hp, m.n1 * hp, tw, PlainColOp<T>{U, U, invM}, st))) return rc;
         const unsigned gf = grid_for(hc, 256, 1 << 16);
+        constexpr bool PHI = sizeof(T) == 8;
         if (hi)
-            hipLaunchKernelGGL((k_sm_filter_fwd<T, true>), dim3(gf), dim3(256), 0, st, U, P.spec3, hc, m.n1, nh, hp, kt, fl, a1e2, s2);
+            hipLaunchKernelGGL((k_sm_filter_fwd<T, true, PHI>), dim3(gf), dim3(256), 0, st, U, P.spec3, hc, m.n1, nh, hp, kt, fl, a1e2, s2);
         else
-            hipLaunchKernelGGL((k_sm_filter_fwd<T, false>), dim3(gf), dim3(256), 0, st, U, P.spec3, hc, m.n1, nh, hp, kt, fl, a1e2, s2);
-        for (int d = 0; d < 3; d++)
+            hipLaunchKernelGGL((k_sm_filter_fwd<T, false, PHI>), dim3(gf), dim3(256), 0, st, U, P.spec3, hc, m.n1, nh, hp, kt, fl, a1e2, s2);
+        for (int d = 0; d < (PHI ? 1 : 3); d++)
             if ((rc = colpass<T, +1>(m.n0, m.n1, nh, hp, m.n1 * hp, tw, PlainColOp<T>{P.spec3 + d * hc, P.spec3 + d * hc, T(1)}, st))) return rc;
     }
     // 4. inverse y passes (3 force spectra as 3*N0 planes) and z c2r into F
-    if (fft_mesh_pow2(m)) {  // phi = inverse transform of P (x pass output in slot 0), F = -grad6(phi)
+    if (layer_one_mesh<T>(m)) {  // phi = inverse transform of P (x pass output in slot 0), F = -grad6(phi)
         T* phi = P.mesh3;
         if ((rc = colpass<T, +1>(m.n1, m.n0, nh, m.n1 * hp, hp, tw, PlainColOp<T>{P.spec3, P.spec3, T(1)}, st))) return rc;
         if ((rc = zpass_c2r<T>(nrows, m.n2, tw, HalfRowLoad<T>{P.spec3, hp}, RealRowStore<T>{phi, m.n2, T(1)}, st, nullptr)))
@@ -1454,11 +1473,10 @@ static int sm_layer_bwd(int kind, const T* pos, const ldl_pos_desc* pdesc, int64
                             reuse ? reinterpret_cast<const unsigned*>(bins) : nullptr, rho, 1.0 / fact, gmax)))
         return rc;
     const KTabs<T> kt = build_tables<T>(P.tabs, m, pdesc->box, st);
-    // 2. unnormalised r2c: power-of-two meshes transform the real-space
-    // divergence of the three meshes (one spectrum, slot 0); others the three
-    // meshes (z and y passes; the filter kernel applies the i D_d)
-    const bool p2 = fft_mesh_pow2(m);
-    if (p2) {
+    // 2. unnormalised r2c of the real-space divergence of the three meshes
+    // (layer_one_mesh: one spectrum, slot 0), else of the three meshes (z and y
+    // passes; the filter kernel applies the i D_d)
+    if (layer_one_mesh<T>(m)) {
         T* dv = reinterpret_cast<T*>(P.spec3 + 2 * hc);  // a real mesh in the free third spectrum
         launch_div6<T>(m, P.mesh3, dv, (T)((double)m.n0 / (60.0 * pdesc->box[0])), (T)((double)m.n1 / (60.0 * pdesc->box[1])),
                        (T)((double)m.n2 / (60.0 * pdesc->box[2])), st);
@@ -1503,15 +1521,16 @@ static int sm_layer_bwd(int kind, const T* pos, const ldl_pos_desc* pdesc, int64
                                    S, m.n2, zdbl, kt, fl, a1e2, gkh, gkl, cpot, prm[0], (int)alpha_rule, s2, P.part);
         });
     } else {
-        for (int d = 0; d < 3; d++)
+        constexpr bool PHI = sizeof(T) == 8;
+        for (int d = 0; d < (PHI ? 1 : 3); d++)
             if ((rc = colpass<T, -1>(m.n0, m.n1, nh, hp, m.n1 * hp, tw, PlainColOp<T>{P.spec3 + d * hc, P.spec3 + d * hc, T(1)}, st))) return rc;
         const unsigned gf = grid_for(hc, 256, 4096);
         ntx = gf;
         if (hi)
-            hipLaunchKernelGGL((k_sm_filter_bwd<T, true>), dim3(gf), dim3(256), 0, st, P.spec3, U, S, hc, m.n1, nh, hp, m.n2, zdbl, kt, fl, a1e2,
+            hipLaunchKernelGGL((k_sm_filter_bwd<T, true, PHI>), dim3(gf), dim3(256), 0, st, P.spec3, U, S, hc, m.n1, nh, hp, m.n2, zdbl, kt, fl, a1e2,
                                gkh, gkl, cpot, prm[0], (int)alpha_rule, s2, P.part);
         else
-            hipLaunchKernelGGL((k_sm_filter_bwd<T, false>), dim3(gf), dim3(256), 0, st, P.spec3, U, S, hc, m.n1, nh, hp, m.n2, zdbl, kt, fl, a1e2,
+            hipLaunchKernelGGL((k_sm_filter_bwd<T, false, PHI>), dim3(gf), dim3(256), 0, st, P.spec3, U, S, hc, m.n1, nh, hp, m.n2, zdbl, kt, fl, a1e2,
                                gkh, gkl, cpot, prm[0], (int)alpha_rule, s2, P.part);
         if ((rc = colpass<T, +1>(m.n0, m.n1, nh, hp, m.n1 * hp, tw, PlainColOp<T>{S, S, T(1)}, st))) return rc;
     }
