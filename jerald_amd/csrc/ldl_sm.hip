@@ -301,21 +301,14 @@ template <typename T> struct Tri3RowLoad {
 
 
 // Rows taken component-fastest (Tri3RowLoad) into the interleaved field F3i
-// (x, y, z packed per cell): the power-of-two z pass hands over whole threes
-// of rows (store3, two cells per call); the any-length pass single rows
-// (store2).
+// (x, y, z packed per cell): the z pass hands over whole threes of rows, two
+// cells per call.
 template <typename T> struct Tri3Store3 {
     static constexpr int NR = 0;
     static constexpr int TRIPLE = 1;
     T* out;
     int64_t n2;
     __device__ __forceinline__ void reduce_out(int64_t, const double*) const {}
-    __device__ __forceinline__ void store2(int64_t R, int m, c2<T> v, double*) const {
-        const int64_t r = R / 3;
-        T* o = out + 3 * (r * n2 + 2 * m) + (R - 3 * r);
-        o[0] = v.x;
-        o[3] = v.y;
-    }
     __device__ __forceinline__ void store3(int64_t r, int m, c2<T> a, c2<T> b, c2<T> c) const {
         T* o = out + 3 * (r * n2 + 2 * m);  // two adjacent cells: 6 consecutive values
         o[0] = a.x;
