@@ -109,6 +109,13 @@ __device__ __forceinline__ int flat_mod(uint64_t e) {
     return (int)(s % 3u);
 }
 
+// *slot = max(*slot, v), for the one maximum of many workgroups: the device
+// atomic only when v exceeds the value read, as one address takes some 80
+// atomics a us.
+template <typename U> __device__ __forceinline__ void raise_max(U* slot, U v) {
+    if (v > __hip_atomic_load(slot, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(slot, v);
+}
+
 // header[c] = bits of max |mass[:, c]| (as double); positive doubles order
 // like their bit patterns, so an integer atomicMax is exact and order free.
 // The (np, NC) array is read flat as coalesced 16-byte vectors of W = 16 /
@@ -170,7 +177,7 @@ __global__ void __launch_bounds__(256) k_absmax(const T* __restrict__ mass, int6
     if (threadIdx.x < NC) {
         const int c = threadIdx.x;
         const double v = fmax(fmax(wmax[c][0], wmax[c][1]), fmax(wmax[c][2], wmax[c][3]));
-        if (v > 0.0) atomicMax(&hdr[c], (unsigned long long)__double_as_longlong(v));
+        if (v > 0.0) raise_max(&hdr[c], (unsigned long long)__double_as_longlong(v));
     }
 }
 
@@ -206,7 +213,7 @@ __global__ void __launch_bounds__(256) k_mesh_absmax(const T* __restrict__ w, in
     __syncthreads();
     if (threadIdx.x == 0) {
         const double b = fmax(fmax(wm[0], wm[1]), fmax(wm[2], wm[3]));
-        if (b > 0.0) atomicMax(slot, (unsigned long long)__double_as_longlong(b));
+        if (b > 0.0) raise_max(slot, (unsigned long long)__double_as_longlong(b));
     }
 }
 
@@ -1165,7 +1172,7 @@ __global__ void __launch_bounds__(TB) k_paint_tiles(const T* __restrict__ pos, P
                 float b = wmx[0];
 #pragma unroll
                 for (int i = 1; i < TB / 64; i++) b = fmaxf(b, wmx[i]);
-                atomicMax(vmax, __float_as_uint(b));  // non-negative floats order like their bits
+                raise_max(vmax, __float_as_uint(b));  // non-negative floats order like their bits
             }
         }
     }

@@ -774,12 +774,9 @@ __device__ __forceinline__ void block_absmax3(const T (&mx)[3], unsigned long lo
     }
     __syncthreads();
     if (threadIdx.x < 3) {
-        // the maxima of the many workgroups are alike: an atomic only when this
-        // one exceeds the current value keeps the three addresses uncontended
         const int c = threadIdx.x;
         const double v = fmax(fmax(wm[c][0], wm[c][1]), fmax(wm[c][2], wm[c][3]));
-        const unsigned long long b = (unsigned long long)__double_as_longlong(v);
-        if (v > 0.0 && b > *reinterpret_cast<volatile unsigned long long*>(&gmax[c])) atomicMax(&gmax[c], b);
+        if (v > 0.0) raise_max(&gmax[c], (unsigned long long)__double_as_longlong(v));
     }
 }
 
