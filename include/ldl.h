@@ -92,10 +92,12 @@ int ldl_buildplan(const int64_t nmesh[3], int32_t out[2]);
 
 /* ----------------------------------------------------------------- paint */
 /* Workspace for a paint of ``ncomp`` (1 or 3) components of ``np`` particles
- * with paint ``flags``: the particle sort's keys and indices (12 B per
- * particle plus 8 B per 8x16x32-cell tile); LDL_PAINT_DIRECT adds the 64-bit
- * accumulator mesh (8 B per cell and component); LDL_PAINT_FLOAT_ATOMIC needs
- * none (0). */
+ * with paint ``flags``: the particle sort's keys and indices (8 B per particle
+ * plus 64 B per 8x16x32-cell tile) and, from 2^22 particles on, its lists of
+ * particles out of order (12 B per particle and up to 8 MB; a smaller workspace
+ * without room for them is accepted: the sort then does without);
+ * LDL_PAINT_DIRECT adds the 64-bit accumulator mesh (8 B per cell and
+ * component); LDL_PAINT_FLOAT_ATOMIC needs none (0). */
 size_t ldl_paint_workspace_bytes(const int64_t nmesh[3], int32_t ncomp, int64_t np, int32_t flags);
 
 /* Replaces ppaint_f32/_f64 (lib/cpu.cc:51-72 -> lib/parops_fast.h:483-531).
