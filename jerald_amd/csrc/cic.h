@@ -344,8 +344,8 @@ __device__ __forceinline__ void gather8(const T* __restrict__ F, const Stencil<T
     }
 }
 
-// ---- power-of-two meshes (every FFT mesh: axes 2^k <= 1024, at most 2^30
-// cells): 32-bit byte offsets from a uniform base pointer, wraps by masking.
+// ---- meshes of at most 4 GB: 32-bit byte offsets from a uniform base pointer
+// (power-of-two ones, axes 2^k, wrap by masking).
 struct MeshP2 {
     uint32_t msk[3];   // n - 1 per axis
     uint32_t lg1, lg2;  // log2 n1, log2 n2
@@ -367,13 +367,26 @@ template <typename T> struct StencilP2 {
     T f[3];
 };
 
-// LU: lattice positions with unit steps and power-of-two strides
-// (PosDec::lattice_unit_p2), decoded without run-time branches.
-template <typename T, bool LU = false>
+// Position decode of the gathers, and of the paint's sort and deposit kernels
+// (which must use the same one), chosen on the host: any positions on any mesh
+// (sides below 2^31); any on a power-of-two mesh; on a power-of-two mesh lattice
+// positions with unit steps and power-of-two strides (PosDec::lattice_unit_p2);
+// absolute positions on a power-of-two and on any mesh.  The last three decode
+// without run-time branches on the form, which keeps their kernels' registers
+// down (FP32 absolute positions, 384^3: key pass 99 VGPRs, 300 us decoding any
+// form, 76 and 188 us; 1-component deposit 87, 503 us, and 64, 326 us).
+constexpr int kDecAny = 0, kDecP2 = 1, kDecLU = 2, kDecPhysP2 = 3, kDecPhys = 4;
+constexpr bool dec_p2(int dm) { return dm == kDecP2 || dm == kDecLU || dm == kDecPhysP2; }
+template <typename T> inline int decode_mode(const PosDec<T>& pd, bool p2) {
+    if (pd.physical()) return p2 ? kDecPhysP2 : kDecPhys;
+    return !p2 ? kDecAny : pd.lattice_unit_p2() ? kDecLU : kDecP2;
+}
+
+template <typename T, int DM>
 __device__ __forceinline__ void locate_p2(const PosDec<T>& pd, const MeshP2& mp, T x0, T x1, T x2, int64_t p, StencilP2<T>& st) {
     uint32_t idx[3];
-    if constexpr (LU) pd.decode_lu(x0, x1, x2, p, mp.msk, idx, st.f);
-    else pd.decode_p2(x0, x1, x2, p, mp.msk, idx, st.f);
+    if constexpr (DM == kDecLU) pd.decode_lu(x0, x1, x2, p, mp.msk, idx, st.f);
+    else pd.template decode_p2<DM == kDecPhysP2>(x0, x1, x2, p, mp.msk, idx, st.f);
     const uint32_t i1 = (idx[0] + 1u) & mp.msk[0], j1 = (idx[1] + 1u) & mp.msk[1];
     constexpr uint32_t lb = sizeof(T) == 4 ? 2 : 3;
     st.row[0] = ((idx[0] << mp.lg1) | idx[1]) << (mp.lg2 + lb);
@@ -383,13 +396,13 @@ __device__ __forceinline__ void locate_p2(const PosDec<T>& pd, const MeshP2& mp,
     st.k = idx[2];
 }
 
-// Corner values of NF fields on a power-of-two mesh: one two-element load per
-// (field, row) -- z-adjacent corners are contiguous -- all issued before any
-// is used; lanes with k = N2 - 1 load the pair ending at k and then the wrapped
-// corner (N2 >= 2).
+// Corner values of NF fields: one two-element load per (field, row) --
+// z-adjacent corners are contiguous -- all issued before any is used; lanes
+// with k = last = N2 - 1 load the pair ending at k and then the wrapped corner
+// (N2 >= 2).
 template <typename T, int NF>
-__device__ __forceinline__ void gather_p2(const T* const (&F)[NF], const StencilP2<T>& st, const MeshP2& mp, T (&v)[NF][8]) {
-    const bool wrap = st.k == mp.msk[2];
+__device__ __forceinline__ void gather_32(const T* const (&F)[NF], const StencilP2<T>& st, uint32_t last, T (&v)[NF][8]) {
+    const bool wrap = st.k == last;
     const uint32_t kb = (wrap ? st.k - 1u : st.k) * (uint32_t)sizeof(T);
     Pair<T> pr[NF][4];
 #pragma unroll
@@ -437,8 +450,32 @@ __device__ __forceinline__ Cell3<T> load_cell3(const T* p) {
     return Cell3<T>{{p[0], p[1], p[2]}};
 }
 
+// The 8 corners of all components of an interleaved field: rows' byte offsets
+// are the 1-slot ones times 3, formed in 32 bits, or in 64 (W) where the field
+// exceeds 4 GB.
+template <typename T, bool W>
+__device__ __forceinline__ void gather3i_32(const T* __restrict__ F3i, const StencilP2<T>& st, uint32_t last, T (&v)[3][8]) {
+    using Off = typename std::conditional<W, uint64_t, uint32_t>::type;
+    const uint32_t k0 = st.k * (uint32_t)sizeof(T), k1 = st.k == last ? 0u : k0 + (uint32_t)sizeof(T);
+    const char* b = reinterpret_cast<const char*>(F3i);
+    Cell3<T> a[4], c[4];
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+        a[r] = load_cell3(reinterpret_cast<const T*>(b + (Off)(st.row[r] + k0) * 3u));
+        c[r] = load_cell3(reinterpret_cast<const T*>(b + (Off)(st.row[r] + k1) * 3u));
+    }
+#pragma unroll
+    for (int r = 0; r < 4; r++)
+#pragma unroll
+        for (int q = 0; q < 3; q++) {
+            v[q][2 * r] = a[r].v[q];
+            v[q][2 * r + 1] = c[r].v[q];
+        }
+}
+
 // Mesh geometry policies of the gather kernels: GeomAny works on every mesh;
-// GeomP2 on power-of-two meshes whose byte size fits 32 bits (p2_ok).
+// GeomP2 on power-of-two meshes and GeomN on others whose fields' byte sizes
+// fit 32 bits (fits_32), both with W for interleaved fields beyond that.
 template <typename T> struct GeomAny {
     using St = Stencil<T>;
     Mesh m;
@@ -464,57 +501,68 @@ template <typename T> struct GeomAny {
         }
     }
 };
-template <typename T, bool LU = false> struct GeomP2 {
+template <typename T, int DM, bool W> struct GeomP2 {
     using St = StencilP2<T>;
     MeshP2 mp;
     __device__ __forceinline__ void locate(const PosDec<T>& pd, T x0, T x1, T x2, int64_t p, St& st) const {
-        locate_p2<T, LU>(pd, mp, x0, x1, x2, p, st);
+        locate_p2<T, DM>(pd, mp, x0, x1, x2, p, st);
     }
     template <int NF>
-    __device__ __forceinline__ void gather(const T* const (&F)[NF], const St& st, T (&v)[NF][8]) const { gather_p2<T, NF>(F, st, mp, v); }
-    // the three components of an interleaved field; byte offsets are the
-    // 1-slot row offsets times 3, so the field's bytes must fit 32 bits (p2_ok3i)
+    __device__ __forceinline__ void gather(const T* const (&F)[NF], const St& st, T (&v)[NF][8]) const { gather_32<T, NF>(F, st, mp.msk[2], v); }
     __device__ __forceinline__ void gather3i(const T* __restrict__ F3i, const St& st, T (&v)[3][8]) const {
-        constexpr uint32_t cb = 3 * sizeof(T);
-        const uint32_t k0 = st.k * cb, k1 = ((st.k + 1u) & mp.msk[2]) * cb;
-        const char* b = reinterpret_cast<const char*>(F3i);
-        Cell3<T> a[4], c[4];
-#pragma unroll
-        for (int r = 0; r < 4; r++) {
-            a[r] = load_cell3(reinterpret_cast<const T*>(b + (st.row[r] * 3u + k0)));
-            c[r] = load_cell3(reinterpret_cast<const T*>(b + (st.row[r] * 3u + k1)));
-        }
-#pragma unroll
-        for (int r = 0; r < 4; r++)
-#pragma unroll
-            for (int q = 0; q < 3; q++) {
-                v[q][2 * r] = a[r].v[q];
-                v[q][2 * r + 1] = c[r].v[q];
-            }
+        gather3i_32<T, W>(F3i, st, mp.msk[2], v);
     }
 };
+template <typename T, bool PHYS, bool W> struct GeomN {
+    using St = StencilP2<T>;
+    uint32_t n0, n1, n2;
+    __device__ __forceinline__ void locate(const PosDec<T>& pd, T x0, T x1, T x2, int64_t p, St& st) const {
+        uint32_t id[3];
+        pd.template decode_32<PHYS>(x0, x1, x2, p, id, st.f);
+        const uint32_t i1 = id[0] + 1u == n0 ? 0u : id[0] + 1u, j1 = id[1] + 1u == n1 ? 0u : id[1] + 1u;
+        const uint32_t b = n2 * (uint32_t)sizeof(T);
+        st.row[0] = (id[0] * n1 + id[1]) * b;
+        st.row[1] = (id[0] * n1 + j1) * b;
+        st.row[2] = (i1 * n1 + id[1]) * b;
+        st.row[3] = (i1 * n1 + j1) * b;
+        st.k = id[2];
+    }
+    template <int NF>
+    __device__ __forceinline__ void gather(const T* const (&F)[NF], const St& st, T (&v)[NF][8]) const { gather_32<T, NF>(F, st, n2 - 1u, v); }
+    __device__ __forceinline__ void gather3i(const T* __restrict__ F3i, const St& st, T (&v)[3][8]) const {
+        gather3i_32<T, W>(F3i, st, n2 - 1u, v);
+    }
+};
+// one field's byte size fits 32 bits (then every side is below 2^31)
 template <typename T>
-inline bool p2_ok(const Mesh& m) {
-    return is_pow2(m.n0) && is_pow2(m.n1) && is_pow2(m.n2) && m.n2 >= 2 &&
-           m.cells() * (int64_t)sizeof(T) <= (int64_t(1) << 32);
+inline bool fits_32(const Mesh& m) {
+    return m.n2 >= 2 && m.cells() * (int64_t)sizeof(T) <= (int64_t(1) << 32);
 }
-// Calls f(geom) with the fastest policy that fits the mesh and the positions.
-template <typename T, typename Fn>
+inline bool mesh_pow2(const Mesh& m) { return is_pow2(m.n0) && is_pow2(m.n1) && is_pow2(m.n2); }
+// Calls f(geom) with the fastest policy that fits the mesh and the positions
+// (layer forward gather, 384^3 FP32 absolute positions: GeomAny 0.604 ms, GeomN
+// 0.578; the backward one at 100^3: 29.5 and 25.4 us; position gradients of a
+// paint on 225 x 180 x 150 FP64: 96 and 85 us).
+template <typename T, bool W = false, typename Fn>
 inline void with_geom(const Mesh& m, const PosDec<T>& pd, Fn&& f) {
-    if (p2_ok<T>(m) && pd.lattice_unit_p2()) f(GeomP2<T, true>{mesh_p2(m)});
-    else if (p2_ok<T>(m)) f(GeomP2<T>{mesh_p2(m)});
-    else f(GeomAny<T>{m});
+    if (!fits_32<T>(m)) {
+        f(GeomAny<T>{m});
+        return;
+    }
+    const uint32_t n0 = (uint32_t)m.n0, n1 = (uint32_t)m.n1, n2 = (uint32_t)m.n2;
+    switch (decode_mode(pd, mesh_pow2(m))) {
+        case kDecAny: f(GeomN<T, false, W>{n0, n1, n2}); break;
+        case kDecPhys: f(GeomN<T, true, W>{n0, n1, n2}); break;
+        case kDecP2: f(GeomP2<T, kDecP2, W>{mesh_p2(m)}); break;
+        case kDecPhysP2: f(GeomP2<T, kDecPhysP2, W>{mesh_p2(m)}); break;
+        default: f(GeomP2<T, kDecLU, W>{mesh_p2(m)}); break;
+    }
 }
 // Same for kernels that also gather an interleaved 3-component field.
-template <typename T>
-inline bool p2_ok3i(const Mesh& m) {
-    return p2_ok<T>(m) && m.cells() * 3 * (int64_t)sizeof(T) <= (int64_t(1) << 32);
-}
 template <typename T, typename Fn>
 inline void with_geom3i(const Mesh& m, const PosDec<T>& pd, Fn&& f) {
-    if (p2_ok3i<T>(m) && pd.lattice_unit_p2()) f(GeomP2<T, true>{mesh_p2(m)});
-    else if (p2_ok3i<T>(m)) f(GeomP2<T>{mesh_p2(m)});
-    else f(GeomAny<T>{m});
+    if (m.cells() * 3 * (int64_t)sizeof(T) <= (int64_t(1) << 32)) with_geom<T, false>(m, pd, f);
+    else with_geom<T, true>(m, pd, f);
 }
 
 // value (deriv < 0) or derivative along ``deriv`` (box units)
@@ -648,26 +696,13 @@ inline TileGeom make_tiles(const Mesh& m, const int sh[3]) {
     return g;
 }
 
-// Position decode of the paint's sort and deposit kernels, chosen on the host
-// (both kernels use the same one): any mesh; a power-of-two mesh; a
-// power-of-two mesh with lattice positions of unit steps and power-of-two
-// strides (PosDec::lattice_unit_p2), decoded without run-time branches.
-constexpr int kDecAny = 0, kDecP2 = 1, kDecLU = 2;
-
 // Lower CIC corner (32-bit cell indices) and fractions of particle p: on a
 // power-of-two mesh with mask wraps, else with the general decode.
 template <typename T, int DM>
 __device__ __forceinline__ void cell_of(const PosDec<T>& pd, const MeshP2& mp, T x0, T x1, T x2, int64_t p, uint32_t id[3], T f[3]) {
-    if constexpr (DM == kDecLU) {
-        pd.decode_lu(x0, x1, x2, p, mp.msk, id, f);
-    } else if constexpr (DM == kDecP2) {
-        pd.decode_p2(x0, x1, x2, p, mp.msk, id, f);
-    } else {
-        int64_t idx[3];
-        pd.decode_xyz(x0, x1, x2, p, idx, f);
-#pragma unroll
-        for (int d = 0; d < 3; d++) id[d] = (uint32_t)idx[d];
-    }
+    if constexpr (DM == kDecLU) pd.decode_lu(x0, x1, x2, p, mp.msk, id, f);
+    else if constexpr (dec_p2(DM)) pd.template decode_p2<DM == kDecPhysP2>(x0, x1, x2, p, mp.msk, id, f);
+    else pd.template decode_32<DM == kDecPhys>(x0, x1, x2, p, id, f);
 }
 
 // Sort key of a particle whose CIC lower corner is cell id: 8 * tile + face
@@ -682,14 +717,14 @@ __device__ __forceinline__ unsigned tile_key(const uint32_t id[3], const TileGeo
 #pragma unroll
     for (int d = 0; d < 3; d++) {
         t[d] = id[d] >> tg.sh[d];
-        if constexpr (DM == kDecAny) {
+        if constexpr (!dec_p2(DM)) {
             const uint32_t hi = (t[d] + 1u) << tg.sh[d];  // one past the tile's last cell
             if (id[d] + 1u == (hi < tg.n32[d] ? hi : tg.n32[d])) fc |= 1u << d;
         } else {
             if (((id[d] + 1u) & tg.fm[d]) == 0u) fc |= 1u << d;
         }
     }
-    if constexpr (DM == kDecAny) return (((t[0] * (unsigned)tg.nt[1] + t[1]) * (unsigned)tg.nt[2] + t[2]) << 3) | fc;
+    if constexpr (!dec_p2(DM)) return (((t[0] * (unsigned)tg.nt[1] + t[1]) * (unsigned)tg.nt[2] + t[2]) << 3) | fc;
     else return (((((t[0] << tg.lnt[1]) | t[1]) << tg.lnt[2]) | t[2]) << 3) | fc;
 }
 
@@ -1155,10 +1190,13 @@ __global__ void __launch_bounds__(256) k_bin_scatter(int64_t np, const unsigned*
 // 2^g > 2 W + 1, so a cell's |sum| stays below 2^29 plus 4 per contribution:
 // the int32 sums equal the int64 ones of the same deposits.
 //
+// The FP32 one-component deposit is held to 64 VGPRs (four workgroups per CU)
+// for the decodes that need no more than one spilled register for it.
+//
 // vmax (FP32, one component, may be NULL): max |cell| of the painted mesh, as
 // FP32 bits, by one atomicMax per workgroup into a zeroed slot.
 template <typename T, int NC, int TX, int TY, int TZ, int TB, int DM, bool ACC32 = false>
-__global__ void __launch_bounds__(TB) k_paint_tiles(const T* __restrict__ pos, PosDec<T> pd, int64_t np, const T* __restrict__ mass,
+__global__ void __launch_bounds__(TB, (NC == 1 && sizeof(T) == 4 && DM >= kDecLU ? 8 : 1)) k_paint_tiles(const T* __restrict__ pos, PosDec<T> pd, int64_t np, const T* __restrict__ mass,
                                                      T mscalar, Mesh m, MeshP2 mp, TileGeom tg, const unsigned* __restrict__ offsets,
                                                      const unsigned* __restrict__ sorted, const unsigned long long* __restrict__ hdr,
                                                      double scale, T* __restrict__ out, unsigned* __restrict__ vmax = nullptr) {

@@ -173,15 +173,16 @@ int paint_impl(const T* pos, const ldl_pos_desc* pdesc, int64_t np, const T* mas
     const int64_t nk = tg.nkeys();
     if (m.n0 >= (1ll << 31) || m.n1 >= (1ll << 31) || m.n2 >= (1ll << 31) || nk >= (1ll << 32))
         return fail(LDL_EUNSUPPORTED, "the tiled paint takes mesh axes below 2^31 cells and fewer than 2^29 tiles");
-    // power-of-two meshes decode with 32-bit mask wraps, unit-step lattice
-    // positions with power-of-two strides without run-time branches (the sort
-    // and deposit kernels must use the same decode)
-    const bool p2 = is_pow2(m.n0) && is_pow2(m.n1) && is_pow2(m.n2);
-    const int dm = !p2 ? kDecAny : pd.lattice_unit_p2() ? kDecLU : kDecP2;
+    // (the sort and deposit kernels must use the same decode)
+    const int dm = decode_mode(pd, mesh_pow2(m));
     auto with_dm = [dm](auto&& f) {
-        if (dm == kDecLU) f(std::integral_constant<int, kDecLU>{});
-        else if (dm == kDecP2) f(std::integral_constant<int, kDecP2>{});
-        else f(std::integral_constant<int, kDecAny>{});
+        switch (dm) {
+            case kDecLU: f(std::integral_constant<int, kDecLU>{}); break;
+            case kDecP2: f(std::integral_constant<int, kDecP2>{}); break;
+            case kDecPhysP2: f(std::integral_constant<int, kDecPhysP2>{}); break;
+            case kDecPhys: f(std::integral_constant<int, kDecPhys>{}); break;
+            default: f(std::integral_constant<int, kDecAny>{}); break;
+        }
     };
     const MeshP2 mp = mesh_p2(m);
     auto* counts = reinterpret_cast<unsigned*>(wb + w.counts);
@@ -205,7 +206,7 @@ int paint_impl(const T* pos, const ldl_pos_desc* pdesc, int64_t np, const T* mas
         offsets = const_cast<unsigned*>(bins_in);
         sorted = const_cast<unsigned*>(bins_in) + nk + 1;
     } else {
-        const bool strays = w.strays && pd.kind == LDL_POS_PHYSICAL;
+        const bool strays = w.strays && pd.physical();
         const int64_t nz = nk + (strays ? kBins : 0), nchunks = sort_chunks(np);
         hipLaunchKernelGGL(k_fill<unsigned>, dim3(grid_for(nz, kBlock, 1 << 16)), dim3(kBlock), 0, st, counts, nz, 0u);
         StrayLists sl{};
@@ -219,7 +220,7 @@ int paint_impl(const T* pos, const ldl_pos_desc* pdesc, int64_t np, const T* mas
             KTimer _t("paint_bin", st);
             with_dm([&](auto D) {
                 constexpr int DM = decltype(D)::value;
-                if constexpr (DM != kDecLU) {  // (a lattice decode never has lists)
+                if constexpr (DM == kDecPhysP2 || DM == kDecPhys) {
                     if (strays) {
                         hipLaunchKernelGGL((k_bin_keys<T, kSortPPT, DM, true>), gb, dim3(256), 0, st, pos, pd, np, mp, tg, counts, key, sl);
                         return;

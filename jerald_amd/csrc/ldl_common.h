@@ -61,12 +61,41 @@ __host__ __device__ __forceinline__ int64_t wrapi(int64_t i, int64_t n) {
     return r < 0 ? r + n : r;
 }
 
+// a / b, correctly rounded as the IEEE division, for positive normal b and y =
+// RN(1 / b): two corrections of a y with exact residuals (Markstein, IBM J.
+// Res. Dev. 34, 1990: one from a faithful quotient rounds correctly; the first
+// makes it faithful).  Five operations instead of the division's dozen.  Tiny
+// a, whose residuals could underflow, and y = 0 divide.
+template <typename T> __device__ __forceinline__ T div_by_cell(T a, T b, T y) {
+    constexpr T tiny = sizeof(T) == 4 ? T(1e-25) : T(1e-250);
+    if (!(a >= tiny) || y == T(0)) return a / b;
+    T q = a * y;
+    q = fma(fma(-b, q, a), y, q);
+    return fma(fma(-b, q, a), y, q);
+}
+
+// fmod(|r|, b) with the sign of r, b > 0: exact as fmod is (each difference of
+// two numbers within a factor of two is), in a few instructions a binary digit
+// of |r| / b; NaN for an infinite r.  The library's loop costs a kernel some 20
+// registers.
+template <typename T> __device__ __forceinline__ T fmod_digits(T r, T b) {
+    T a = fabs(r);
+    if (!(a < T(INFINITY))) return T(NAN);
+    while (a >= b) {
+        T s = ldexp(b, ilogb(a) - ilogb(b));
+        if (s > a) s *= T(0.5);
+        a -= s;
+    }
+    return copysign(a, r);
+}
+
 // ------------------------------------------------------ position decoding
 // Device-side copy of ldl_pos_desc, specialised to the working precision.
 template <typename T> struct PosDec {
     int kind;
     T box[3];
     T cell[3];     // box / N in T (reference: BoxSize / Nmesh in the working dtype)
+    T cellrcp[3];  // 1 / cell, rounded to T (0: outside div_by_cell's range)
     T cellinv[3];  // N / box in T (reference: Nmesh[d] / BoxSize[d], lib/parops_fast.h:748-750)
     uint32_t l12, l2;  // lattice strides (Np < 2^32 for the lattice form)
     int sh12, sh2;     // log2 of the strides when they are powers of two, else -1
@@ -84,23 +113,26 @@ template <typename T> struct PosDec {
     // Mesh coordinates x (before the floor) of particle p from its loaded
     // coordinates, and the integer cell offset ``base`` they are relative to
     // (the lattice cell; 0 for physical positions).
-    template <typename I>
+    // PHYS: known to be physical.
+    template <bool PHYS, typename I>
     __device__ __forceinline__ void coords(T x0, T x1, T x2, int64_t p, T x[3], I base[3]) const {
         x[0] = x0;
         x[1] = x1;
         x[2] = x2;
         base[0] = base[1] = base[2] = 0;
-        if (kind == LDL_POS_PHYSICAL) {
+        if (PHYS || kind == LDL_POS_PHYSICAL) {
 #pragma unroll
             for (int d = 0; d < 3; d++) {
                 // numpy remainder semantics, then division (jaxpops_bind.py:163-164);
-                // fmod is the identity on [0, L)
+                // fmod is the identity on [0, L), exactly r - L on [L, 2L)
+                // and the identity again on (-L, 0), where L is added
                 T r = x[d];
                 if (!(r >= T(0) && r < box[d])) {
-                    r = fmod(r, box[d]);
-                    if (r != T(0) && ((r < T(0)) != (box[d] < T(0)))) r += box[d];
+                    if (r >= box[d] && r < T(2) * box[d]) r -= box[d];
+                    else if (!(r > -box[d] && r < T(0))) r = fmod_digits(r, box[d]);
+                    if (r < T(0)) r += box[d];
                 }
-                x[d] = r / cell[d];
+                x[d] = div_by_cell(r, cell[d], cellrcp[d]);
             }
         } else {
             uint32_t pp = (uint32_t)p;
@@ -135,7 +167,7 @@ template <typename T> struct PosDec {
     __device__ __forceinline__ void decode_xyz(T x0, T x1, T x2, int64_t p, int64_t idx[3], T f[3]) const {
         T x[3];
         int64_t base[3];
-        coords(x0, x1, x2, p, x, base);
+        coords<false>(x0, x1, x2, p, x, base);
 #pragma unroll
         for (int d = 0; d < 3; d++) {
             T fl = floor(x[d]);
@@ -144,12 +176,43 @@ template <typename T> struct PosDec {
         }
     }
 
+    // Same, 32-bit cell indices (sides below 2^31).
+    template <bool PHYS>
+    __device__ __forceinline__ void decode_32(T x0, T x1, T x2, int64_t p, uint32_t idx[3], T f[3]) const {
+        T x[3];
+        uint32_t base[3];
+        coords<PHYS>(x0, x1, x2, p, x, base);
+#pragma unroll
+        for (int d = 0; d < 3; d++) {
+            const T fl = floor(x[d]);
+            f[d] = x[d] - fl;
+            if constexpr (PHYS) {  // 0 <= fl <= n (or NaN, which converts to 0)
+                const uint32_t u = (uint32_t)(int32_t)fl;
+                idx[d] = u < (uint32_t)n[d] ? u : 0u;
+            } else {
+                idx[d] = wrap_cell(fl, base[d], n[d]);
+            }
+        }
+    }
+    // base + fl wrapped into [0, n), base < n: in 32 bits up to one period off
+    // (a negative sum wraps to 2^31 or more, above every n), else as wrapi.
+    static __device__ __forceinline__ uint32_t wrap_cell(T fl, uint32_t base, int64_t n) {
+        if (fabs(fl) < T(1 << 29)) {
+            const uint32_t u = base + (uint32_t)(int32_t)fl, m = (uint32_t)n;
+            if (u < m) return u;
+            const uint32_t v = fl < T(0) ? u + m : u - m;
+            if (v < m) return v;
+        }
+        return (uint32_t)wrapi((int64_t)base + (int64_t)fl, n);
+    }
+
     // Power-of-two mesh: 32-bit cell indices wrapped with the masks n - 1
     // (mesh coordinates within +-2^31 cells).
+    template <bool PHYS>
     __device__ __forceinline__ void decode_p2(T x0, T x1, T x2, int64_t p, const uint32_t msk[3], uint32_t idx[3], T f[3]) const {
         T x[3];
         int32_t base[3];
-        coords(x0, x1, x2, p, x, base);
+        coords<PHYS>(x0, x1, x2, p, x, base);
 #pragma unroll
         for (int d = 0; d < 3; d++) {
             T fl = floor(x[d]);
@@ -172,6 +235,7 @@ template <typename T> struct PosDec {
             idx[d] = (uint32_t)(base[d] + (int32_t)fl) & msk[d];
         }
     }
+    bool physical() const { return kind == LDL_POS_PHYSICAL; }
     bool lattice_unit_p2() const { return kind == LDL_POS_LATTICE && unit && sh12 >= 0 && sh2 >= 0; }
 };
 
@@ -185,6 +249,8 @@ inline int make_posdec(const ldl_pos_desc* pd, const int64_t nmesh[3], int64_t n
         if (!(pd->box[d] > 0.0) || !std::isfinite(pd->box[d])) return fail(LDL_EINVAL, "box sizes must be positive and finite");
         out->box[d] = (T)pd->box[d];
         out->cell[d] = out->box[d] / (T)nmesh[d];
+        constexpr double span = sizeof(T) == 4 ? 1e12 : 1e100;
+        out->cellrcp[d] = (double)out->cell[d] > 1 / span && (double)out->cell[d] < span ? T(1) / out->cell[d] : T(0);
         out->cellinv[d] = (T)nmesh[d] / out->box[d];
         out->n[d] = nmesh[d];
         out->lstep[d] = pd->lattice_step[d];
@@ -278,14 +344,14 @@ __device__ __forceinline__ int64_t xcd_tile_rev(int64_t bid, int64_t nb) {
 // A workgroup takes chunks of kChunk consecutive particles (one per thread);
 // its chunk id comes from xcd_tile, so each XCD owns a contiguous run of chunk
 // ids.  Linear order: chunk c starts at particle c * kChunk.  Blocked order,
-// for a lattice of L0 x L1 x L2 particles stored in lattice order with L2 a
-// multiple of kChunk: chunk ids run over slabs of S lattice planes (S = L0 / 8
-// when 8 divides L0, so each XCD owns one slab), then blocks of J rows, then
-// the S planes, then the J rows, then the L2 / kChunk chunks of a row.  The
-// mesh rows a lattice plane gathers from are reused by the next plane J rows'
-// worth of particles later, while they are still in the XCD's L2; in linear
-// order that reuse distance is a whole lattice plane, whose mesh footprint
-// (several fields of 2-3 mesh planes) exceeds the L2.
+// for a lattice of L0 x L1 x L2 particles stored in lattice order: chunk ids
+// run over slabs of S lattice planes (S = L0 / 8 when 8 divides L0, so each XCD
+// owns one slab), then blocks of J rows (a multiple of kChunk particles), then
+// the S planes, then the block's H chunks.  The mesh rows a lattice plane
+// gathers from are reused by the next plane a block's worth of particles
+// later, while they are still in the XCD's L2; in linear order that reuse
+// distance is a whole lattice plane, whose mesh footprint (several fields of
+// 2-3 mesh planes) exceeds the L2.
 constexpr int kChunk = 256;
 struct Sweep {
     int blocked;
@@ -295,10 +361,9 @@ struct Sweep {
         if (!blocked) return c * kChunk;
         uint32_t q = (uint32_t)c;
         const uint32_t h = q % H; q /= H;
-        const uint32_t jj = q % J; q /= J;
         const uint32_t i = q % S; q /= S;
         const uint32_t yb = q % NYB, slab = q / NYB;
-        return (((int64_t)(slab * S + i) * L1 + yb * J + jj) * L2) + (int64_t)h * kChunk;
+        return (((int64_t)(slab * S + i) * L1 + yb * J) * L2) + (int64_t)h * kChunk;
     }
 };
 
@@ -308,16 +373,17 @@ inline Sweep make_sweep(const PosDec<T>& pd, int64_t np) {
     w.nchunks = (np + kChunk - 1) / kChunk;
     if (pd.kind != LDL_POS_LATTICE || np == 0) return w;
     const int64_t L2 = pd.l2, L1 = pd.l12 / pd.l2, L0 = np / pd.l12;
-    if (L2 % kChunk) return w;
+    int64_t J = 0;  // 32 rows or the most below
+    for (int64_t j = 32; j >= 2 && !J; j >>= 1)
+        if (L1 % j == 0 && j * L2 % kChunk == 0) J = j;
+    if (!J) return w;
     w.blocked = 1;
     w.L1 = (uint32_t)L1;
     w.L2 = (uint32_t)L2;
-    w.H = (uint32_t)(L2 / kChunk);
-    w.J = (uint32_t)L1;
-    for (int64_t j = 32; j >= 2; j >>= 1)
-        if (L1 % j == 0) { w.J = (uint32_t)j; break; }
+    w.J = (uint32_t)J;
+    w.H = (uint32_t)(J * L2 / kChunk);
     w.S = (uint32_t)(L0 % 8 == 0 ? L0 / 8 : L0);
-    w.NYB = (uint32_t)(L1 / w.J);
+    w.NYB = (uint32_t)(L1 / J);
     return w;
 }
 
