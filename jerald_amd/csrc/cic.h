@@ -5,7 +5,7 @@
 #include <cstring>
 #include <type_traits>
 
-#include "ldl_common.h"
+#include "axis.h"
 
 namespace ldl {
 
@@ -83,10 +83,6 @@ __device__ __forceinline__ void deposits_of(const T f[3], DepositT<T> M, Deposit
 template <typename T>
 __device__ __forceinline__ void deposits(const T f[3], T m, int s, DepositT<T> q[8]) {
     deposits_of<T>(f, fixed_mass<T>(m, s), q);
-}
-
-static __global__ void k_copy_u64(const unsigned long long* __restrict__ src, unsigned long long* __restrict__ dst, int64_t n) {
-    for (int64_t i = threadIdx.x; i < n; i += blockDim.x) dst[i] = src[i];
 }
 
 static __global__ void k_fill_u64(unsigned long long* __restrict__ p, int64_t n, unsigned long long v) {
@@ -1423,11 +1419,43 @@ __global__ void __launch_bounds__(TB, (NC == 1 && sizeof(T) == 4 && DM >= kDecLU
     }
 }
 
-// slot (FP32 bits of max |w| from the 1-component paint that wrote w) -> the
-// double bits k_mesh_absmax would give for w and scale: (double)max|w| * scale.
-static __global__ void k_vmax_scaled(const unsigned* __restrict__ slot, double scale, unsigned long long* __restrict__ out) {
-    const double v = (double)__uint_as_float(*slot) * scale;
-    if (v > 0.0) *out = (unsigned long long)__double_as_longlong(v);
+// Everything a paint sets before its first pass, and the axis tables of the
+// layer it is part of, in one launch (each launch of a few values costs some 5
+// us of a small mesh's pass): the header (hbits in every slot; max |mass| per
+// component copied from absmax_in, which is cleared if ``reset``; slot 3 the
+// largest cell weight sum, (double)max|w| * wscale, from the FP32 bits the
+// 1-component paint that wrote w recorded), the recorded maximum's own slot and
+// the sort's counters.
+struct PaintPrep {
+    unsigned long long* hdr;
+    unsigned long long hbits;
+    unsigned long long* absmax_in;
+    int nc, reset;
+    const unsigned* vmax_in;
+    double wscale;
+    unsigned* vmax_out;
+    unsigned* counts;
+    int64_t ncounts;
+};
+constexpr int kHdrSlots = 32;
+template <typename T>
+__global__ void __launch_bounds__(256) k_paint_prep(PaintPrep a, AxisTabs<T> tabs) {
+    const int64_t tid = blockIdx.x * (int64_t)256 + threadIdx.x, nth = (int64_t)gridDim.x * 256;
+    for (int64_t i = tid; i < a.ncounts; i += nth) a.counts[i] = 0u;
+    for (int64_t i = tid; i < tabs.total(); i += nth) tabs.entry(i);
+    if (tid < kHdrSlots) {
+        unsigned long long v = a.hbits;
+        if (a.absmax_in && tid < a.nc) {
+            v = a.absmax_in[tid];
+            if (a.reset) a.absmax_in[tid] = 0ull;
+        }
+        if (tid == 3 && a.vmax_in) {
+            const double w = (double)__uint_as_float(*a.vmax_in) * a.wscale;
+            if (w > 0.0) v = (unsigned long long)__double_as_longlong(w);
+        }
+        if (a.hdr) a.hdr[tid] = v;
+        if (tid == 0 && a.vmax_out) *a.vmax_out = 0u;
+    }
 }
 
 size_t paint_ws_bytes(const Mesh& m, int nc, int64_t np, int32_t flags);
@@ -1436,7 +1464,8 @@ template <typename T>
 int paint_impl(const T* pos, const ldl_pos_desc* pdesc, int64_t np, const T* mass, double mscalar, int nc,
                const int64_t nmesh[3], double out_scale, int32_t flags, T* out, void* ws, size_t ws_bytes,
                hipStream_t st, unsigned* bins_out = nullptr, const unsigned* bins_in = nullptr, const T* wmesh = nullptr,
-               double wscale = 0.0, const unsigned long long* absmax_in = nullptr);
+               double wscale = 0.0, unsigned long long* absmax_in = nullptr, bool absmax_reset = false,
+               const AxisTabs<T>& tabs = AxisTabs<T>{});
 // Particle sort by tile and face class that a 1-component paint can
 // hand to a later 3-component paint of the same positions: offsets
 // (8 ntiles + 1), sorted particle indices (np), then (FP32) the FP32 bits of

@@ -95,7 +95,7 @@ template <typename T>
 int paint_impl(const T* pos, const ldl_pos_desc* pdesc, int64_t np, const T* mass, double mscalar, int nc,
                const int64_t nmesh[3], double out_scale, int32_t flags, T* out, void* ws, size_t ws_bytes,
                hipStream_t st, unsigned* bins_out, const unsigned* bins_in, const T* wmesh, double wscale,
-               const unsigned long long* absmax_in) {
+               unsigned long long* absmax_in, bool absmax_reset, const AxisTabs<T>& tabs) {
     Mesh m;
     int rc = check_mesh(nmesh, &m);
     if (rc) return rc;
@@ -110,7 +110,13 @@ int paint_impl(const T* pos, const ldl_pos_desc* pdesc, int64_t np, const T* mas
     const unsigned gp = grid_for(np, kBlock, 1 << 16);
     const unsigned gm = grid_for(tot, kBlock, 1 << 16);
     const int mode = flags & 1;
+    auto prep = [&](const PaintPrep& a) {
+        const int64_t n = std::max<int64_t>(std::max<int64_t>(a.ncounts, tabs.total()), 1);
+        hipLaunchKernelGGL(k_paint_prep<T>, dim3(grid_for(n, kBlock, 1 << 12)), dim3(kBlock), 0, st, a, tabs);
+    };
     if (mode == LDL_PAINT_FLOAT_ATOMIC) {
+        if (tabs.total() || (absmax_in && absmax_reset))
+            prep(PaintPrep{nullptr, 0, absmax_reset ? absmax_in : nullptr, nc, 1, nullptr, 0.0, nullptr, nullptr, 0});
         hipLaunchKernelGGL(k_fill<T>, dim3(gm), dim3(kBlock), 0, st, out, tot, T(0));
         if (np > 0) {
             if (nc == 1)
@@ -136,10 +142,11 @@ int paint_impl(const T* pos, const ldl_pos_desc* pdesc, int64_t np, const T* mas
         double a = std::fabs((double)(T)mscalar);
         std::memcpy(&hbits, &a, 8);
     }
-    hipLaunchKernelGGL(k_fill_u64, dim3(1), dim3(64), 0, st, hdr, (int64_t)(kHdrBytes / 8), hbits);
-    if (mass && absmax_in) {  // max |m| per component handed over by the kernel that wrote the masses
-        hipLaunchKernelGGL(k_copy_u64, dim3(1), dim3(64), 0, st, absmax_in, hdr, (int64_t)nc);
-    } else if (mass && np > 0) {
+    static_assert(kHdrSlots * 8 == kHdrBytes, "the header's slots fill it");
+    if (!mass) absmax_in = nullptr;  // max |m| per component may be handed over by the kernel that wrote the masses
+    PaintPrep pp{hdr, hbits, absmax_in, nc, absmax_reset, nullptr, 0.0, nullptr, nullptr, 0};
+    auto absmax = [&]() {
+        if (!mass || absmax_in || np == 0) return;
         KTimer _t("paint_absmax", st);
         // two workgroups per CU keep 8 MB of loads in flight; more of them, all
         // ending at once, only queue on the maximum's address (3.4e6 FP64
@@ -147,8 +154,10 @@ int paint_impl(const T* pos, const ldl_pos_desc* pdesc, int64_t np, const T* mas
         const dim3 ga(grid_for((np * nc * (int64_t)sizeof(T) + 63) / 64, kBlock, 512));
         if (nc == 1) hipLaunchKernelGGL((k_absmax<T, 1>), ga, dim3(kBlock), 0, st, mass, np, hdr);
         else hipLaunchKernelGGL((k_absmax<T, 3>), ga, dim3(kBlock), 0, st, mass, np, hdr);
-    }
+    };
     if (flags & LDL_PAINT_DIRECT) {
+        prep(pp);
+        absmax();
         // reference variant: one device-scope 64-bit atomic per corner
         if (!(flags & LDL_PAINT_WS_ZEROED))
             hipLaunchKernelGGL(k_fill_u64, dim3(gm), dim3(kBlock), 0, st, acc, tot, 0ull);
@@ -197,18 +206,25 @@ int paint_impl(const T* pos, const ldl_pos_desc* pdesc, int64_t np, const T* mas
     if (bins_out) {
         offsets = bins_out;
         sorted = bins_out + nk + 1;
-        if (nc == 1 && sizeof(T) == 4) {
-            vmax_out = bins_out + nk + 1 + np;
-            hipLaunchKernelGGL(k_fill<unsigned>, dim3(1), dim3(64), 0, st, vmax_out, (int64_t)1, 0u);
-        }
+        if (nc == 1 && sizeof(T) == 4) vmax_out = bins_out + nk + 1 + np;
     }
+    const bool strays = w.strays && pd.physical();
+    pp.vmax_out = vmax_out;
+    if (!bins_in) {
+        pp.counts = counts;
+        pp.ncounts = nk + (strays ? kBins : 0);
+    } else if (nc == 3 && sizeof(T) == 4 && wmesh) {
+        // recorded by the 1-component paint that wrote the sort and wmesh
+        pp.vmax_in = bins_in + nk + 1 + np;
+        pp.wscale = wscale;
+    }
+    prep(pp);
+    absmax();
     if (bins_in) {
         offsets = const_cast<unsigned*>(bins_in);
         sorted = const_cast<unsigned*>(bins_in) + nk + 1;
     } else {
-        const bool strays = w.strays && pd.physical();
-        const int64_t nz = nk + (strays ? kBins : 0), nchunks = sort_chunks(np);
-        hipLaunchKernelGGL(k_fill<unsigned>, dim3(grid_for(nz, kBlock, 1 << 16)), dim3(kBlock), 0, st, counts, nz, 0u);
+        const int64_t nchunks = sort_chunks(np);
         StrayLists sl{};
         if (strays) {
             auto u = [&](size_t off) { return reinterpret_cast<unsigned*>(wb + off); };
@@ -236,7 +252,7 @@ int paint_impl(const T* pos, const ldl_pos_desc* pdesc, int64_t np, const T* mas
         {
             KTimer _t("paint_scan", st);
             const unsigned nseg = (unsigned)((nk + kScanSeg - 1) / kScanSeg);
-            hipLaunchKernelGGL(k_scan_sums, dim3(nseg), dim3(1024), 0, st, counts, nk, segsum);
+            if (nseg > 1) hipLaunchKernelGGL(k_scan_sums, dim3(nseg), dim3(1024), 0, st, counts, nk, segsum);
             hipLaunchKernelGGL(k_scan_apply, dim3(nseg), dim3(1024), 0, st, counts, nk, segsum, offsets, counts);  // counts become the cursors
         }
         if (np > 0) {
@@ -255,9 +271,7 @@ int paint_impl(const T* pos, const ldl_pos_desc* pdesc, int64_t np, const T* mas
         });
     } else if (sizeof(T) == 4 && wmesh) {
         // FP32 with the positions' unit-mass density known: 32-bit accumulators
-        if (bins_in) {  // recorded by the 1-component paint that wrote the sort and wmesh
-            hipLaunchKernelGGL(k_vmax_scaled, dim3(1), dim3(1), 0, st, bins_in + nk + 1 + np, wscale, hdr + 3);
-        } else {
+        if (!bins_in) {
             KTimer _t("paint_absmax", st);
             hipLaunchKernelGGL(k_mesh_absmax<T>, dim3(grid_for(cells, kBlock, 512)), dim3(kBlock), 0, st, wmesh, cells, wscale, hdr + 3);
         }
@@ -323,9 +337,9 @@ int readout_impl(const T* pos, const ldl_pos_desc* pdesc, int64_t np, const T* f
 }
 
 template int paint_impl<float>(const float*, const ldl_pos_desc*, int64_t, const float*, double, int, const int64_t*, double, int32_t, float*, void*,
-                               size_t, hipStream_t, unsigned*, const unsigned*, const float*, double, const unsigned long long*);
+                               size_t, hipStream_t, unsigned*, const unsigned*, const float*, double, unsigned long long*, bool, const AxisTabs<float>&);
 template int paint_impl<double>(const double*, const ldl_pos_desc*, int64_t, const double*, double, int, const int64_t*, double, int32_t, double*,
-                                void*, size_t, hipStream_t, unsigned*, const unsigned*, const double*, double, const unsigned long long*);
+                                void*, size_t, hipStream_t, unsigned*, const unsigned*, const double*, double, unsigned long long*, bool, const AxisTabs<double>&);
 template int readout_impl<float>(const float*, const ldl_pos_desc*, int64_t, const float*, const int64_t*, int, int, const float*, float*, hipStream_t);
 template int readout_impl<double>(const double*, const ldl_pos_desc*, int64_t, const double*, const int64_t*, int, int, const double*, double*, hipStream_t);
 

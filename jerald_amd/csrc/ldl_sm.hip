@@ -40,32 +40,6 @@ static constexpr int kBlk = 256;
 static_assert(kBlk == kChunk, "gathers take one particle per thread");
 
 // ---------------------------------------------------------------- tables
-// Per-axis wavenumbers k = 2 pi fftfreq(N, cell) (pmesh.py:174-186; the z
-// axis keeps N/2+1 entries, so its last one is -pi/cell) and the 6th-order
-// finite-difference gradient symbol (45 sin kD - 9 sin 2kD + sin 3kD)/(30 D)
-// (model.py:200-201), evaluated in FP64.
-template <typename T> struct AxisTabs {
-    T* k[3];
-    T* D[3];
-    int64_t n[3], count[3];
-    double cell[3];
-};
-template <typename T>
-__global__ void k_axis_tables(AxisTabs<T> a) {
-    int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    int d = 0;  // the three axes' tables, one after the other
-    while (d < 2 && i >= a.count[d]) i -= a.count[d++];
-    if (i >= a.count[d]) return;
-    const int64_t n = a.n[d];
-    const double cell = a.cell[d];
-    T* __restrict__ k = a.k[d];
-    T* __restrict__ D = a.D[d];
-    const int64_t m = 2 * i < n ? i : i - n;  // fftfreq order, odd n included: 0..(n-1)/2, -(n-1)/2..-1
-    const double th = 2.0 * (double)m / (double)n;  // k cell / pi
-    k[i] = (T)(2.0 * M_PI * (double)m / ((double)n * cell));
-    D[i] = (T)((45.0 * sinpi(th) - 9.0 * sinpi(2.0 * th) + sinpi(3.0 * th)) / (30.0 * cell));
-}
-
 template <typename T> struct KTabs {
     const T* k[3];
     const T* D[3];
@@ -182,77 +156,103 @@ static SmPtrs<T> sm_ptrs(void* ws, const SmWs& w) {
     return p;
 }
 
+// The axis tables of a mesh in ``tabs``: what fills them and what reads them.
 template <typename T>
-static KTabs<T> build_tables(T* tabs, const Mesh& m, const double box[3], hipStream_t st) {
+static KTabs<T> axis_tables(T* tabs, const Mesh& m, const double box[3], AxisTabs<T>* a) {
     const int64_t cnt[3] = {m.n0, m.n1, m.nh()};
     const int64_t nn[3] = {m.n0, m.n1, m.n2};
     KTabs<T> kt;
-    AxisTabs<T> a;
     T* p = tabs;
     for (int d = 0; d < 3; d++) {
-        a.k[d] = p;
-        a.D[d] = p + cnt[d];
-        a.n[d] = nn[d];
-        a.count[d] = cnt[d];
-        a.cell[d] = box[d] / (double)nn[d];
-        kt.k[d] = a.k[d];
-        kt.D[d] = a.D[d];
+        a->k[d] = p;
+        a->D[d] = p + cnt[d];
+        a->n[d] = nn[d];
+        a->count[d] = cnt[d];
+        a->cell[d] = box[d] / (double)nn[d];
+        kt.k[d] = a->k[d];
+        kt.D[d] = a->D[d];
         p += 2 * cnt[d];
     }
-    hipLaunchKernelGGL(k_axis_tables<T>, dim3(grid_for(cnt[0] + cnt[1] + cnt[2], kBlk)), dim3(kBlk), 0, st, a);
+    return kt;
+}
+template <typename T>
+static KTabs<T> build_tables(T* tabs, const Mesh& m, const double box[3], hipStream_t st) {
+    AxisTabs<T> a;
+    const KTabs<T> kt = axis_tables<T>(tabs, m, box, &a);
+    hipLaunchKernelGGL(k_axis_tables<T>, dim3(grid_for(a.total(), 256)), dim3(256), 0, st, a);
     return kt;
 }
 
 // Sum column j of a (nblocks x stride) FP64 array and add it to out[map[j]]
-// (or store when ``assign``); fixed order, one workgroup.
+// (or store when ``assign``); fixed order, one workgroup of 1024.
 struct RedMap {
     int n;
     int map[12];
 };
-// One pass over the rows: thread t sums column j of rows t, t + 256, ... in
-// that order, then the waves and the four wave sums in a fixed order.  Four
-// rows' loads are issued before they are added (in the same order).
-__global__ void __launch_bounds__(256) k_reduce_cols(const double* __restrict__ part, int64_t nblocks, int stride, RedMap rm,
-                                                     double* __restrict__ out, int assign) {
-    constexpr int MX = 12, U = 4;
-    __shared__ double red[MX][4];
-    double s[MX];
+struct RedJob {
+    const double* part;
+    int64_t nblocks;
+    int stride;
+    RedMap rm;
+    double* out;
+    int assign;
+};
+constexpr int kRedCols = 12, kRedThreads = 1024;
+// One pass over the rows: thread t sums column j of rows t, t + 1024, ... in
+// that order, then the waves and the wave sums in a fixed order.  Four rows'
+// loads are issued before they are added (in the same order).  tot[j] (shared)
+// holds the totals after a barrier.
+__device__ __forceinline__ void reduce_cols(const double* __restrict__ part, int64_t nblocks, int stride, int n, double (&red)[kRedCols][kRedThreads / 64],
+                                            double (&tot)[kRedCols]) {
+    constexpr int U = 4;
+    double s[kRedCols];
 #pragma unroll
-    for (int j = 0; j < MX; j++) s[j] = 0.0;
+    for (int j = 0; j < kRedCols; j++) s[j] = 0.0;
     int64_t b = threadIdx.x;
-    for (; b + (U - 1) * 256 < nblocks; b += U * 256) {
-        double v[U][MX];
+    for (; b + (U - 1) * kRedThreads < nblocks; b += U * kRedThreads) {
+        double v[U][kRedCols];
 #pragma unroll
         for (int u = 0; u < U; u++)
 #pragma unroll
-            for (int j = 0; j < MX; j++) v[u][j] = j < rm.n ? part[(b + u * 256) * stride + j] : 0.0;
+            for (int j = 0; j < kRedCols; j++) v[u][j] = j < n ? part[(b + u * kRedThreads) * stride + j] : 0.0;
 #pragma unroll
         for (int u = 0; u < U; u++)
 #pragma unroll
-            for (int j = 0; j < MX; j++)
-                if (j < rm.n) s[j] += v[u][j];
+            for (int j = 0; j < kRedCols; j++)
+                if (j < n) s[j] += v[u][j];
     }
-    for (; b < nblocks; b += 256) {
+    for (; b < nblocks; b += kRedThreads) {
         const double* row = part + b * stride;
 #pragma unroll
-        for (int j = 0; j < MX; j++)
-            if (j < rm.n) s[j] += row[j];
+        for (int j = 0; j < kRedCols; j++)
+            if (j < n) s[j] += row[j];
     }
 #pragma unroll
-    for (int j = 0; j < MX; j++) {
-        if (j < rm.n) {
+    for (int j = 0; j < kRedCols; j++) {
+        if (j < n) {
             const double v = wave_sum(s[j]);
             if ((threadIdx.x & 63) == 0) red[j][threadIdx.x >> 6] = v;
         }
     }
     __syncthreads();
-    if ((int)threadIdx.x < rm.n) {
-        const int j = threadIdx.x;
-        const double t = (red[j][0] + red[j][1]) + (red[j][2] + red[j][3]);
-        if (assign) out[rm.map[j]] = t;
-        else out[rm.map[j]] += t;
+    if ((int)threadIdx.x < n) {
+        double t = 0.0;
+        for (int w = 0; w < kRedThreads / 64; w++) t += red[threadIdx.x][w];
+        tot[threadIdx.x] = t;
+    }
+    __syncthreads();
+}
+// Workgroup 0 does a, workgroup 1 (if launched) b.
+__global__ void __launch_bounds__(kRedThreads) k_reduce_cols(RedJob a, RedJob b) {
+    __shared__ double red[kRedCols][kRedThreads / 64], tot[kRedCols];
+    const RedJob& r = blockIdx.x ? b : a;
+    reduce_cols(r.part, r.nblocks, r.stride, r.rm.n, red, tot);
+    if ((int)threadIdx.x < r.rm.n) {
+        double* o = r.out + r.rm.map[threadIdx.x];
+        *o = r.assign ? tot[threadIdx.x] : *o + tot[threadIdx.x];
     }
 }
+static void launch_reduce(hipStream_t st, const RedJob& a) { hipLaunchKernelGGL(k_reduce_cols, dim3(1), dim3(kRedThreads), 0, st, a, RedJob{}); }
 
 // --------------------------------------------------------- z-pass functors
 template <typename T> struct PowRowLoad {  // (rho + 1e-8)^gamma, model.py:193
@@ -1193,7 +1193,12 @@ template <typename T, bool PLAIN = false> struct LossSq2Store {
 };
 
 // out = {loss / npix, g_mu, g_w, g_b, loss_v / npix_v[, g_zs]}
-__global__ void k_loss_finish(const double* __restrict__ sums, const double* __restrict__ npix, double* __restrict__ out, int nout) {
+// The loss columns' totals, and out = {loss, dL/dmu, dL/dw, dL/db, validation
+// loss (HI: , dL/dzs)} from them.
+__global__ void __launch_bounds__(kRedThreads) k_loss_finish(const double* __restrict__ part, int64_t nblocks, const double* __restrict__ npix,
+                                                             double* __restrict__ out, int nout) {
+    __shared__ double red[kRedCols][kRedThreads / 64], sums[kRedCols];
+    reduce_cols(part, nblocks, kLossCols, kLossCols, red, sums);
     if (threadIdx.x == 0) {
         out[0] = sums[0] / npix[0];
         out[1] = sums[1];
@@ -1202,6 +1207,10 @@ __global__ void k_loss_finish(const double* __restrict__ sums, const double* __r
         out[4] = npix[1] > 0.0 ? sums[4] / npix[1] : 0.0;
         if (nout > 5) out[5] = sums[5];
     }
+}
+__global__ void k_npix(double* npix, double cells) {
+    npix[0] = cells;
+    npix[1] = 0.0;
 }
 
 // ------------------------------------------------------- HI depletion
@@ -1358,11 +1367,12 @@ static int sm_layer_fwd(int kind, const T* pos, const ldl_pos_desc* pdesc, int64
     // these positions wrote into bins)
     const bool tiled = !(pflags & (LDL_PAINT_FLOAT_ATOMIC | LDL_PAINT_DIRECT));
     const bool bins_in = tiled && bins && (pflags & LDL_PAINT_BINS_VALID);
+    AxisTabs<T> at;  // filled by the paint's first launch
+    const KTabs<T> kt = axis_tables<T>(P.tabs, m, pdesc->box, &at);
     if ((rc = paint_impl<T>(pos, pdesc, np, nullptr, 1.0, 1, nmesh, fact, pflags & ~LDL_PAINT_BINS_VALID, rho, P.paint, w.paint, st,
                             tiled && !bins_in ? reinterpret_cast<unsigned*>(bins) : nullptr,
-                            bins_in ? reinterpret_cast<const unsigned*>(bins) : nullptr)))
+                            bins_in ? reinterpret_cast<const unsigned*>(bins) : nullptr, nullptr, 0.0, nullptr, false, at)))
         return rc;
-    const KTabs<T> kt = build_tables<T>(P.tabs, m, pdesc->box, st);
     // half spectra: nh columns in rows of pitch hp, hc apart
     const int64_t nrows = m.n0 * m.n1, nh = m.nh(), hp = spec_pitch<T>(m), hc = spec_cells<T>(m);
     c2<T>* U = reinterpret_cast<c2<T>*>(Ubuf);
@@ -1459,10 +1469,13 @@ static int sm_layer_bwd(int kind, const T* pos, const ldl_pos_desc* pdesc, int64
     // 1. gF_d = paint(X, g_d)  (3 meshes in mesh3)
     const bool reuse = bins && !(pflags & (LDL_PAINT_FLOAT_ATOMIC | LDL_PAINT_DIRECT));
     // (the forward density rho = fact * sum of CIC weights bounds the cells' sums)
+    // gmax has served once its values are in the paint's header: cleared there
+    // for the maxima of g_in
+    AxisTabs<T> at;
+    const KTabs<T> kt = axis_tables<T>(P.tabs, m, pdesc->box, &at);
     if ((rc = paint_impl<T>(pos, pdesc, np, gout, 0.0, 3, nmesh, 1.0, pflags, P.mesh3, P.paint, w.paint, st, nullptr,
-                            reuse ? reinterpret_cast<const unsigned*>(bins) : nullptr, rho, 1.0 / fact, gmax)))
+                            reuse ? reinterpret_cast<const unsigned*>(bins) : nullptr, rho, 1.0 / fact, gmax, np > 0, at)))
         return rc;
-    const KTabs<T> kt = build_tables<T>(P.tabs, m, pdesc->box, st);
     // 2. unnormalised r2c of the real-space divergence of the three meshes
     // (layer_one_mesh: one spectrum, slot 0), else of the three meshes (z and y
     // passes; the filter kernel applies the i D_d)
@@ -1527,21 +1540,20 @@ static int sm_layer_bwd(int kind, const T* pos, const ldl_pos_desc* pdesc, int64
     // partial columns -> parameter slots: alpha, kh, kl, nu (HI: then alpha2,
     // kh2, kl2, nu2, gamma2)
     const RedMap rx = hi ? RedMap{9, {0, 2, 3, 4, 5, 7, 8, 9, 6}} : RedMap{4, {0, 2, 3, 4}};
-    hipLaunchKernelGGL(k_reduce_cols, dim3(1), dim3(256), 0, st, P.part, ntx, rx.n, rx, grad, 0);
     // 4. inverse y, z c2r with the gamma-power adjoint -> g_rho (mesh3[0])
     if ((rc = colpass<T, +1>(m.n1, m.n0, nh, m.n1 * hp, hp, tw, PlainColOp<T>{S, S, T(1)}, st))) return rc;
     T* grho = P.mesh3;
     int64_t nzb = 0;
+    double* zpart = P.part + ntx * rx.n;  // after the x pass's partials
     if ((rc = zpass_c2r<T>(nrows, m.n2, tw, HalfRowLoad<T>{S, hp},
-                           GammaBwdStore<T>{rho, grho, m.n2, (T)(1.0 / (double)cells), (T)prm[1], P.part}, st, &nzb,
+                           GammaBwdStore<T>{rho, grho, m.n2, (T)(1.0 / (double)cells), (T)prm[1], zpart}, st, &nzb,
                            "zpass_c2r_gamma")))
         return rc;
     RedMap rz{1, {1}};
-    hipLaunchKernelGGL(k_reduce_cols, dim3(1), dim3(256), 0, st, P.part, nzb, 1, rz, grad, 0);
+    hipLaunchKernelGGL(k_reduce_cols, dim3(2), dim3(kRedThreads), 0, st, RedJob{P.part, ntx, rx.n, rx, grad, 0}, RedJob{zpart, nzb, 1, rz, grad, 0});
     // 5. position adjoint
     if (np > 0)
         {
-            if (gmax) hipLaunchKernelGGL(k_fill_u64, dim3(1), dim3(64), 0, st, gmax, (int64_t)3, 0ull);  // the paint has read it
             KTimer _t("sm_bwd_gather", st);
             with_geom3i<T>(m, pd, [&](auto geo) {
                 hipLaunchKernelGGL((k_sm_bwd_gather<T, decltype(geo)>), dim3(sweep2_grid(sw)), dim3(kBlk), 0, st, pos, pd, np, sw, F, grho, geo,
@@ -1591,17 +1603,17 @@ static int sm_loss(int kind, const T* rho, const T* target, const T* mask, const
     if (!ws || wsb < w.total) return fail(LDL_EINVAL, "sm workspace too small (see ldl_sm_workspace_bytes)");
     const SmPtrs<T> P = sm_ptrs<T>(ws, w);
     const int64_t cells = m.cells();
-    // part layout: [0, 16) npix scratch and sums; block partials from 64
+    // part layout: npix, from 16 the smoothing's field sums; block partials from 64
     double* npix = P.part;          // {npix, npix_v}
-    double* sums = P.part + 8;      // kLossCols sums
     double* bpart = P.part + 64;
     const unsigned gb = 2048;
-    hipLaunchKernelGGL(k_mask_sums<T>, dim3(gb), dim3(256), 0, st, mask, maskv, cells, bpart);
-    RedMap rn{2, {0, 1}};
-    hipLaunchKernelGGL(k_reduce_cols, dim3(1), dim3(256), 0, st, bpart, (int64_t)gb, 2, rn, npix, 1);
-    if (!mask) {  // npix = number of cells
-        const double nc = (double)cells;
-        hipLaunchKernelGGL(k_fill<double>, dim3(1), dim3(1), 0, st, npix, (int64_t)1, nc);
+    if (mask || maskv) {
+        hipLaunchKernelGGL(k_mask_sums<T>, dim3(gb), dim3(256), 0, st, mask, maskv, cells, bpart);
+        RedMap rn{2, {0, 1}};
+        launch_reduce(st, RedJob{bpart, (int64_t)gb, 2, rn, npix, 1});
+        if (!mask) hipLaunchKernelGGL(k_fill<double>, dim3(1), dim3(1), 0, st, npix, (int64_t)1, (double)cells);
+    } else {
+        hipLaunchKernelGGL(k_npix, dim3(1), dim3(1), 0, st, npix, (double)cells);
     }
     RespPar<T> rp{};
     rp.index = (T)index;
@@ -1619,10 +1631,10 @@ static int sm_loss(int kind, const T* rho, const T* target, const T* mask, const
         rp.dep = dep;
         rp.gdep = grho ? gdep : nullptr;
     }
-    RedMap r6{kLossCols, {0, 1, 2, 3, 4, 5, 6}};
+    const int nout = kind == kKindHi ? 6 : 5;
     if (smooth_kind == 0) {
         { KTimer _t("loss", st); hipLaunchKernelGGL(k_loss_direct<T>, dim3(gb), dim3(256), 0, st, rho, target, mask, maskv, rp, cells, npix, grho, bpart); }
-        hipLaunchKernelGGL(k_reduce_cols, dim3(1), dim3(256), 0, st, bpart, (int64_t)gb, kLossCols, r6, sums, 1);
+        hipLaunchKernelGGL(k_loss_finish, dim3(1), dim3(kRedThreads), 0, st, bpart, (int64_t)gb, npix, out, nout);
     } else {
         const c2<T>* tw;
         if ((rc = twiddles<T>(&tw))) return rc;
@@ -1695,7 +1707,7 @@ static int sm_loss(int kind, const T* rho, const T* target, const T* mask, const
         else
             hipLaunchKernelGGL((k_loss_diff<T, false>), dim3(gb), dim3(256), 0, st, rho, target, rp, cells, diff, dpart);
         const RedMap r1{1, {0}};
-        hipLaunchKernelGGL(k_reduce_cols, dim3(1), dim3(256), 0, st, dpart, (int64_t)gb, 1, r1, dsum, 1);
+        launch_reduce(st, RedJob{dpart, (int64_t)gb, 1, r1, dsum, 1});
         if (smooth_kind == 2 && p_norm == 2 && !mask && !maskv && grho) {
             // unmasked L2 with the Gaussian: one smoothing with W^2 = the
             // Gaussian of width sigma sqrt(2) (W(0)^2 = 1) gives the loss and
@@ -1717,16 +1729,15 @@ static int sm_loss(int kind, const T* rho, const T* target, const T* mask, const
                                    st, nullptr, "zpass_c2r_loss")))
                 return rc;
             if (grho) {
-                hipLaunchKernelGGL(k_reduce_cols, dim3(1), dim3(256), 0, st, bpart + 6, nzb, kLossCols, r1, gsum, 1);
+                launch_reduce(st, RedJob{bpart + 6, nzb, kLossCols, r1, gsum, 1});
                 if ((rc = smooth(gds, gsum, smooth_par))) return rc;
                 if ((rc = zpass_c2r<T>(nrows, m.n2, tw, HalfRowLoad<T>{S, hp}, RespBwdStore<T>{rho, grho, rp, m.n2, T(1), bpart, gsum, W0 * invMd},
                                        st, nullptr, "zpass_c2r_resp")))
                     return rc;
             }
         }
-        hipLaunchKernelGGL(k_reduce_cols, dim3(1), dim3(256), 0, st, bpart, nzb, kLossCols, r6, sums, 1);
+        hipLaunchKernelGGL(k_loss_finish, dim3(1), dim3(kRedThreads), 0, st, bpart, nzb, npix, out, nout);
     }
-    hipLaunchKernelGGL(k_loss_finish, dim3(1), dim3(64), 0, st, sums, npix, out, kind == kKindHi ? 6 : 5);
     LDL_LAUNCH_CHECK();
     return LDL_OK;
 }
@@ -1795,7 +1806,7 @@ static int hi_depletion_bwd(const T* star, const c2<T>* Sk, const T* S, const T*
     const unsigned gb = 2048;
     hipLaunchKernelGGL(k_hi_dep_bwd<T>, dim3(gb), dim3(256), 0, st, star, S, gdep, cells, dp, gS, P.part);
     const RedMap re{4, {0, 4, 5, 7}};
-    hipLaunchKernelGGL(k_reduce_cols, dim3(1), dim3(256), 0, st, P.part, (int64_t)gb, 4, re, grad8, 1);
+    launch_reduce(st, RedJob{P.part, (int64_t)gb, 4, re, grad8, 1});
     c2<T>* gh = P.spec3;
     if ((rc = r2c_full<T>(m, tw, RealRowLoad<T>{gS, m.n2}, gh, hp, T(1), st))) return rc;
     const SmFilter<T> fl{(T)prm[1], (T)(1.0 / prm[2]), (T)prm[3], 1};
@@ -1804,7 +1815,7 @@ static int hi_depletion_bwd(const T* star, const c2<T>* Sk, const T* S, const T*
     hipLaunchKernelGGL(k_hi_wgrad<T>, dim3(gf), dim3(256), 0, st, gh, sk, hc, m.n1, nh, hp, m.n2, zdbl, (int)(rule != 0), kt, fl,
                        1.0 / (prm[2] * prm[2]), P.part);
     const RedMap rw{4, {1, 2, 3, 6}};
-    hipLaunchKernelGGL(k_reduce_cols, dim3(1), dim3(256), 0, st, P.part, (int64_t)gf, 4, rw, grad8, 1);
+    launch_reduce(st, RedJob{P.part, (int64_t)gf, 4, rw, grad8, 1});
     LDL_LAUNCH_CHECK();
     return LDL_OK;
 }

@@ -204,7 +204,7 @@ class JERALDModel:
         """Response + loss: out (loss at [0], response gradients, validation
         loss at [4]), g_rho and the HI extras (sfield, g_dep)."""
         dt, dev, nm = self.dtype, self.device, self.nm
-        out = torch.zeros(6, dtype=torch.float64, device=dev)
+        out = torch.empty(6, dtype=torch.float64, device=dev)
         g_rho = torch.empty(nm, dtype=dt, device=dev) if need_grad else None
         ws = self._ws()
         common = (L.ptr(rho), L.ptr(self.target), L.ptr(self.masktrain), L.ptr(self.maskvalid), L.ptr(self.field2))
@@ -306,7 +306,7 @@ class JERALDModel:
         P = st["P"]
         fact = st["fact"]
         g = torch.empty_like(P)
-        gmax = torch.zeros(3, dtype=torch.float64, device=dev)  # max |g| per component, handed from call to call
+        gmax = torch.empty(3, dtype=torch.float64, device=dev)  # max |g| per component, handed from call to call
         L.call(f"ldl_paint_vjp_pos_{L.sfx(dt)}", L.ptr(P), self._pd(), P.shape[0], L.ptr(st["g_rho"]), L.i64x3(nm),
                float(fact), L.ptr(g), L.ptr(gmax), L.stream_ptr(dev))
         k = self.npot
