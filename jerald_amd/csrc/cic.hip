@@ -32,7 +32,6 @@ static constexpr int64_t kHdrBytes = 256;
 // threads per CU (6 waves per SIMD), so one tile's LDS clear and write-out
 // overlap the others' deposits.
 static constexpr int kTileX = 8, kTileY = 16, kTileZ = 32;
-static constexpr int kTileSh[3] = {3, 4, 5};
 static constexpr int kAcc32Block = 512;
 // One component (32 KB of 64-bit accumulators): 512 threads with 4 particles
 // each per round, 62 VGPRs, four workgroups per CU (0.84 ms per 512^3 launch
@@ -49,10 +48,34 @@ static inline size_t al256(size_t b) { return (b + 255) & ~(size_t)255; }
 // order by construction and sort without.
 static constexpr int64_t kStrayMin = 1 << 22;
 static constexpr int kSortPPT = 8;  // particles per thread of the sort's passes: chunks of 2048
+// Below 2^20 particles (512 chunks of 2048, two per CU) chunks of 512 spread
+// the passes over more CUs; key and scatter pass, us: 64^3 9.8 and 8.4 -> 7.5
+// and 6.6, 100^3 12.3 and 9.7 -> 10 and 8.8, FP64 14.8 and 9.5 -> 12 and 8.7.
+// 128^3 takes 15 and 12 either way, 160^3 the scatter 16.6 -> 18.6.
+static constexpr int kFewPPT = 2;
+static constexpr int64_t kFew = 1 << 20;
 static inline int64_t sort_chunks(int64_t np) { return (np + 256 * kSortPPT - 1) / (256 * kSortPPT); }
 // Workgroups of the key pass with lists: two chunks each or more.
 static inline int64_t stray_groups(int64_t np) { return std::max<int64_t>(1, std::min<int64_t>(kSegs, sort_chunks(np) / 2)); }
 static inline int64_t stray_group_size(int64_t np) { return (sort_chunks(np) + stray_groups(np) - 1) / stray_groups(np) * 256 * kSortPPT; }
+
+// A mesh of fewer such tiles than the card has CUs (256) leaves CUs idle, each
+// busy one behind a chain of clear, deposit and write-out; 4 x 8 x 16 cells
+// with 256 threads are eight times the workgroups with a shorter chain each.
+// One and three components, us, large tiles -> small: 64^3 FP32 15 and 22 -> 13
+// and 14, FP64 20 and 36 -> 14 and 22; 80^3 (150 large tiles) 17 and 23 -> 15
+// and 18, FP64 21 and 37 -> 17 and 29; 100^3 (364) 20 and 29 -> 21 and 28 with
+// a longer scan; 128^3 (512) 22 and 33 -> 28 and 40.  From kStrayMin particles
+// on the large tiles stay: the sort's lists and the fixed scratch of the paint
+// without allocation are sized with them.
+static constexpr int kSmallX = 4, kSmallY = 8, kSmallZ = 16, kSmallBlock = 256;
+static TileGeom paint_tiles(const Mesh& m, int64_t np, bool* small = nullptr) {
+    static const int large[3] = {3, 4, 5}, sml[3] = {2, 3, 4};
+    const TileGeom tg = make_tiles(m, large);
+    const bool s = tg.ntiles < 256 && np < kStrayMin;
+    if (small) *small = s;
+    return s ? make_tiles(m, sml) : tg;
+}
 
 // Workspace: header | direct-mode mesh (nc, LDL_PAINT_DIRECT only) | counts
 // and the strays' bins | offsets | segment sums | key | sorted | stray lists
@@ -62,7 +85,7 @@ struct PaintWs {
 };
 static bool paint_direct(int32_t flags) { return (flags & LDL_PAINT_DIRECT) && !(flags & LDL_PAINT_FLOAT_ATOMIC); }
 static PaintWs paint_ws(const Mesh& m, int nc, int64_t np, int32_t flags, bool lists = true) {
-    const TileGeom tg = make_tiles(m, kTileSh);
+    const TileGeom tg = paint_tiles(m, np);
     const int64_t nk = tg.nkeys();
     PaintWs w;
     w.acc = al256((size_t)kHdrBytes);
@@ -87,7 +110,7 @@ size_t paint_ws_bytes(const Mesh& m, int nc, int64_t np, int32_t flags) {
 }
 
 size_t paint_bins_bytes(const Mesh& m, int64_t np) {
-    const TileGeom tg = make_tiles(m, kTileSh);
+    const TileGeom tg = paint_tiles(m, np);
     return (size_t)(tg.nkeys() + 1 + (np < 0 ? 0 : np) + 1) * 4;
 }
 
@@ -178,7 +201,8 @@ int paint_impl(const T* pos, const ldl_pos_desc* pdesc, int64_t np, const T* mas
     // tile sums the tile's cells completely in LDS.  A 3-component paint that
     // is handed the sort of an earlier 1-component paint of the same positions
     // (bins_in) skips the sort.
-    const TileGeom tg = make_tiles(m, kTileSh);
+    bool small;
+    const TileGeom tg = paint_tiles(m, np, &small);
     const int64_t nk = tg.nkeys();
     if (m.n0 >= (1ll << 31) || m.n1 >= (1ll << 31) || m.n2 >= (1ll << 31) || nk >= (1ll << 32))
         return fail(LDL_EUNSUPPORTED, "the tiled paint takes mesh axes below 2^31 cells and fewer than 2^29 tiles");
@@ -224,7 +248,8 @@ int paint_impl(const T* pos, const ldl_pos_desc* pdesc, int64_t np, const T* mas
         offsets = const_cast<unsigned*>(bins_in);
         sorted = const_cast<unsigned*>(bins_in) + nk + 1;
     } else {
-        const int64_t nchunks = sort_chunks(np);
+        const bool few = np < kFew;
+        const int64_t nchunks = few ? (np + 256 * kFewPPT - 1) / (256 * kFewPPT) : sort_chunks(np);
         StrayLists sl{};
         if (strays) {
             auto u = [&](size_t off) { return reinterpret_cast<unsigned*>(wb + off); };
@@ -242,7 +267,8 @@ int paint_impl(const T* pos, const ldl_pos_desc* pdesc, int64_t np, const T* mas
                         return;
                     }
                 }
-                hipLaunchKernelGGL((k_bin_keys<T, kSortPPT, DM, false>), gb, dim3(256), 0, st, pos, pd, np, mp, tg, counts, key, sl);
+                if (few) hipLaunchKernelGGL((k_bin_keys<T, kFewPPT, DM, false>), gb, dim3(256), 0, st, pos, pd, np, mp, tg, counts, key, sl);
+                else hipLaunchKernelGGL((k_bin_keys<T, kSortPPT, DM, false>), gb, dim3(256), 0, st, pos, pd, np, mp, tg, counts, key, sl);
             });
             if (strays) {
                 hipLaunchKernelGGL(k_stray_part, gb, dim3(kStrayThreads), 0, st, key, sl);
@@ -257,37 +283,39 @@ int paint_impl(const T* pos, const ldl_pos_desc* pdesc, int64_t np, const T* mas
         }
         if (np > 0) {
             KTimer _t("paint_scatter", st);
-            hipLaunchKernelGGL(k_bin_scatter<kSortPPT>, dim3(grid_for(nchunks, 1, 1 << 15)), dim3(256), 0, st, np, key, strays ? kStrayBit : 0u, counts,
-                               sorted);
+            const dim3 gs(grid_for(nchunks, 1, 1 << 15));
+            if (few) hipLaunchKernelGGL(k_bin_scatter<kFewPPT>, gs, dim3(256), 0, st, np, key, 0u, counts, sorted);
+            else hipLaunchKernelGGL(k_bin_scatter<kSortPPT>, gs, dim3(256), 0, st, np, key, strays ? kStrayBit : 0u, counts, sorted);
             if (strays) hipLaunchKernelGGL(k_stray_scatter, dim3(1024), dim3(kStrayThreads), 0, st, sl, counts, sorted);
         }
     }
-    const dim3 gt((unsigned)tg.ntiles);
+    if (nc == 3 && sizeof(T) == 4 && wmesh && !bins_in) {
+        KTimer _t("paint_absmax", st);
+        hipLaunchKernelGGL(k_mesh_absmax<T>, dim3(grid_for(cells, kBlock, 512)), dim3(kBlock), 0, st, wmesh, cells, wscale, hdr + 3);
+    }
+    // one workgroup of TB threads per tile; ACC32: FP32 with the positions'
+    // unit-mass density known takes 32-bit accumulators
+    auto deposit = [&](auto NC, auto SM, auto TB, auto ACC32) {
+        constexpr int nc_ = decltype(NC)::value, tb = decltype(SM)::value ? kSmallBlock : decltype(TB)::value;
+        constexpr bool sm = decltype(SM)::value != 0, acc32 = decltype(ACC32)::value != 0;
+        with_dm([&](auto D) {
+            hipLaunchKernelGGL((k_paint_tiles<T, nc_, sm ? kSmallX : kTileX, sm ? kSmallY : kTileY, sm ? kSmallZ : kTileZ, tb, decltype(D)::value, acc32>),
+                               dim3((unsigned)tg.ntiles), dim3(tb), 0, st, pos, pd, np, mass, (T)mscalar, m, mp, tg, offsets, sorted, hdr, out_scale, out,
+                               nc_ == 1 ? vmax_out : nullptr);
+        });
+    };
+    auto sized = [&](auto NC, auto TB, auto ACC32) {
+        if (small) deposit(NC, std::integral_constant<int, 1>{}, TB, ACC32);
+        else deposit(NC, std::integral_constant<int, 0>{}, TB, ACC32);
+    };
+    using std::integral_constant;
+    KTimer _t(nc == 1 ? "paint_deposit1" : "paint_deposit3", st);
     if (nc == 1) {
-        KTimer _t("paint_deposit1", st);
-        with_dm([&](auto D) {
-            hipLaunchKernelGGL((k_paint_tiles<T, 1, kTileX, kTileY, kTileZ, kPaint1Block, decltype(D)::value>), gt, dim3(kPaint1Block), 0, st, pos, pd,
-                               np, mass, (T)mscalar, m, mp, tg, offsets, sorted, hdr, out_scale, out, vmax_out);
-        });
+        sized(integral_constant<int, 1>{}, integral_constant<int, kPaint1Block>{}, integral_constant<int, 0>{});
     } else if (sizeof(T) == 4 && wmesh) {
-        // FP32 with the positions' unit-mass density known: 32-bit accumulators
-        if (!bins_in) {
-            KTimer _t("paint_absmax", st);
-            hipLaunchKernelGGL(k_mesh_absmax<T>, dim3(grid_for(cells, kBlock, 512)), dim3(kBlock), 0, st, wmesh, cells, wscale, hdr + 3);
-        }
-        KTimer _t("paint_deposit3", st);
-        if constexpr (sizeof(T) == 4) {
-            with_dm([&](auto D) {
-                hipLaunchKernelGGL((k_paint_tiles<T, 3, kTileX, kTileY, kTileZ, kAcc32Block, decltype(D)::value, true>), gt, dim3(kAcc32Block), 0, st, pos,
-                                   pd, np, mass, (T)mscalar, m, mp, tg, offsets, sorted, hdr, out_scale, out);
-            });
-        }
+        if constexpr (sizeof(T) == 4) sized(integral_constant<int, 3>{}, integral_constant<int, kAcc32Block>{}, integral_constant<int, 1>{});
     } else {
-        KTimer _t("paint_deposit3", st);
-        with_dm([&](auto D) {
-            hipLaunchKernelGGL((k_paint_tiles<T, 3, kTileX, kTileY, kTileZ, 1024, decltype(D)::value>), gt, dim3(1024), 0, st, pos, pd, np, mass,
-                               (T)mscalar, m, mp, tg, offsets, sorted, hdr, out_scale, out);
-        });
+        sized(integral_constant<int, 3>{}, integral_constant<int, 1024>{}, integral_constant<int, 0>{});
     }
     LDL_LAUNCH_CHECK();
     return LDL_OK;
