@@ -59,22 +59,46 @@ static inline int64_t sort_chunks(int64_t np) { return (np + 256 * kSortPPT - 1)
 static inline int64_t stray_groups(int64_t np) { return std::max<int64_t>(1, std::min<int64_t>(kSegs, sort_chunks(np) / 2)); }
 static inline int64_t stray_group_size(int64_t np) { return (sort_chunks(np) + stray_groups(np) - 1) / stray_groups(np) * 256 * kSortPPT; }
 
-// A mesh of fewer such tiles than the card has CUs (256) leaves CUs idle, each
-// busy one behind a chain of clear, deposit and write-out; 4 x 8 x 16 cells
-// with 256 threads are eight times the workgroups with a shorter chain each.
-// One and three components, us, large tiles -> small: 64^3 FP32 15 and 22 -> 13
-// and 14, FP64 20 and 36 -> 14 and 22; 80^3 (150 large tiles) 17 and 23 -> 15
-// and 18, FP64 21 and 37 -> 17 and 29; 100^3 (364) 20 and 29 -> 21 and 28 with
-// a longer scan; 128^3 (512) 22 and 33 -> 28 and 40.  From kStrayMin particles
-// on the large tiles stay: the sort's lists and the fixed scratch of the paint
-// without allocation are sized with them.
+// Which tiles a paint takes.  A sort handed from one paint to another (bins)
+// is read with the tiles it was written with: both ask with the same mesh,
+// particles and accumulator width.
+//
+// kSplitSmall: a mesh of fewer large tiles than the card has CUs (256) leaves
+// CUs idle, each busy one behind a chain of clear, deposit and write-out;
+// 4 x 8 x 16 cells with 256 threads are eight times the workgroups with a
+// shorter chain each.  One and three components, us, large tiles -> small: 64^3
+// FP32 15 and 22 -> 13 and 14, FP64 20 and 36 -> 14 and 22; 80^3 (150 large
+// tiles) 17 and 23 -> 15 and 18, FP64 21 and 37 -> 17 and 29; 100^3 (364) 20
+// and 29 -> 21 and 28 with a longer scan; 128^3 (512) 22 and 33 -> 28 and 40.
+// From kStrayMin particles on the large tiles stay: the sort's lists and the
+// fixed scratch of the paint without allocation are sized with them.
+//
+// kSplitFlat: 8 x 16 x 16 cells where three components take 64-bit sums (FP64,
+// with the one-component paint that hands its sort over, and the FP32
+// three-component paint without a density).  48 KB instead of 96 KB hold three workgroups of 512
+// threads per CU instead of one of 1024, so that clearing, loading, depositing
+// and writing out of different tiles overlap.  256^3, us: FP64 607 -> 496,
+// FP32 339 -> 281; FP64 one component (256 threads) 223 -> 205.  The 32-bit
+// paints have that occupancy with the longer z runs, and the FP64 one-component
+// paint on its own keeps the workspace it had.  Meshes whose keys would
+// no longer fit the stray lists (FP64 at 1024^3) keep the large tiles, and so
+// does a workspace with no room for twice the keys.
+template <int N> using Int = std::integral_constant<int, N>;
+enum Split { kSplitLarge, kSplitSmall, kSplitFlat };
 static constexpr int kSmallX = 4, kSmallY = 8, kSmallZ = 16, kSmallBlock = 256;
-static TileGeom paint_tiles(const Mesh& m, int64_t np, bool* small = nullptr) {
-    static const int large[3] = {3, 4, 5}, sml[3] = {2, 3, 4};
+static constexpr int kFlatZ = 16, kFlat1Block = 256, kFlat3Block = 512;
+struct PaintTiles {
+    TileGeom tg;
+    Split split;
+};
+static PaintTiles paint_tiles(const Mesh& m, int64_t np, bool wide, bool flat = true) {
+    static const int large[3] = {3, 4, 5}, small[3] = {2, 3, 4}, flats[3] = {3, 4, 4};
     const TileGeom tg = make_tiles(m, large);
-    const bool s = tg.ntiles < 256 && np < kStrayMin;
-    if (small) *small = s;
-    return s ? make_tiles(m, sml) : tg;
+    if (tg.ntiles < 256 && np < kStrayMin) return {make_tiles(m, small), kSplitSmall};
+    if (!wide || !flat) return {tg, kSplitLarge};
+    const TileGeom tf = make_tiles(m, flats);
+    if (tf.nkeys() > ((int64_t)kBins << kBinKeysLog)) return {tg, kSplitLarge};
+    return {tf, kSplitFlat};
 }
 
 // Workspace: header | direct-mode mesh (nc, LDL_PAINT_DIRECT only) | counts
@@ -84,8 +108,7 @@ struct PaintWs {
     bool strays;
 };
 static bool paint_direct(int32_t flags) { return (flags & LDL_PAINT_DIRECT) && !(flags & LDL_PAINT_FLOAT_ATOMIC); }
-static PaintWs paint_ws(const Mesh& m, int nc, int64_t np, int32_t flags, bool lists = true) {
-    const TileGeom tg = paint_tiles(m, np);
+static PaintWs paint_ws(const Mesh& m, int nc, int64_t np, int32_t flags, const TileGeom& tg, bool lists = true) {
     const int64_t nk = tg.nkeys();
     PaintWs w;
     w.acc = al256((size_t)kHdrBytes);
@@ -106,12 +129,13 @@ static PaintWs paint_ws(const Mesh& m, int nc, int64_t np, int32_t flags, bool l
 
 size_t paint_ws_bytes(const Mesh& m, int nc, int64_t np, int32_t flags) {
     if (flags & LDL_PAINT_FLOAT_ATOMIC) return 0;  // float atomics deposit straight into the output
-    return paint_ws(m, nc, np < 0 ? 0 : np, flags).total;
+    np = np < 0 ? 0 : np;
+    return paint_ws(m, nc, np, flags, paint_tiles(m, np, nc == 3).tg).total;
 }
 
 size_t paint_bins_bytes(const Mesh& m, int64_t np) {
-    const TileGeom tg = paint_tiles(m, np);
-    return (size_t)(tg.nkeys() + 1 + (np < 0 ? 0 : np) + 1) * 4;
+    np = np < 0 ? 0 : np;
+    return (size_t)(paint_tiles(m, np, true).tg.nkeys() + 1 + np + 1) * 4;
 }
 
 template <typename T>
@@ -152,9 +176,15 @@ int paint_impl(const T* pos, const ldl_pos_desc* pdesc, int64_t np, const T* mas
     }
     if (np > (int64_t)0xFFFFFFFFll) return fail(LDL_EUNSUPPORTED, "paint supports np < 2^32");
     // a workspace without room for the stray lists (ldl_ppaint_noalloc's fixed
-    // one) sorts without them
-    PaintWs w = paint_ws(m, nc, np, flags);
-    if (ws && ws_bytes < w.total) w = paint_ws(m, nc, np, flags, false);
+    // one) or the flat tiles' keys sorts without them
+    const bool wide = sizeof(T) == 8 ? nc == 3 || bins_in || bins_out : nc == 3 && !wmesh;
+    PaintTiles pt = paint_tiles(m, np, wide);
+    PaintWs w = paint_ws(m, nc, np, flags, pt.tg);
+    if (ws && ws_bytes < w.total) w = paint_ws(m, nc, np, flags, pt.tg, false);
+    if (ws && ws_bytes < w.total && !bins_in && !bins_out) {
+        pt = paint_tiles(m, np, wide, false);
+        w = paint_ws(m, nc, np, flags, pt.tg, false);
+    }
     if (!ws || ws_bytes < w.total) return fail(LDL_EINVAL, "paint workspace too small (see ldl_paint_workspace_bytes)");
     char* wb = reinterpret_cast<char*>(ws);
     auto* hdr = reinterpret_cast<unsigned long long*>(wb);
@@ -201,8 +231,7 @@ int paint_impl(const T* pos, const ldl_pos_desc* pdesc, int64_t np, const T* mas
     // tile sums the tile's cells completely in LDS.  A 3-component paint that
     // is handed the sort of an earlier 1-component paint of the same positions
     // (bins_in) skips the sort.
-    bool small;
-    const TileGeom tg = paint_tiles(m, np, &small);
+    const TileGeom& tg = pt.tg;
     const int64_t nk = tg.nkeys();
     if (m.n0 >= (1ll << 31) || m.n1 >= (1ll << 31) || m.n2 >= (1ll << 31) || nk >= (1ll << 32))
         return fail(LDL_EUNSUPPORTED, "the tiled paint takes mesh axes below 2^31 cells and fewer than 2^29 tiles");
@@ -293,29 +322,40 @@ int paint_impl(const T* pos, const ldl_pos_desc* pdesc, int64_t np, const T* mas
         KTimer _t("paint_absmax", st);
         hipLaunchKernelGGL(k_mesh_absmax<T>, dim3(grid_for(cells, kBlock, 512)), dim3(kBlock), 0, st, wmesh, cells, wscale, hdr + 3);
     }
-    // one workgroup of TB threads per tile; ACC32: FP32 with the positions'
-    // unit-mass density known takes 32-bit accumulators
-    auto deposit = [&](auto NC, auto SM, auto TB, auto ACC32) {
-        constexpr int nc_ = decltype(NC)::value, tb = decltype(SM)::value ? kSmallBlock : decltype(TB)::value;
-        constexpr bool sm = decltype(SM)::value != 0, acc32 = decltype(ACC32)::value != 0;
+    // one workgroup of TB threads per tile of TX x TY x TZ cells; ACC32: FP32
+    // with the positions' unit-mass density known takes 32-bit accumulators
+    auto deposit = [&](auto NC, auto TX, auto TY, auto TZ, auto TB, auto ACC32) {
+        constexpr int nc_ = decltype(NC)::value, tb = decltype(TB)::value;
         with_dm([&](auto D) {
-            hipLaunchKernelGGL((k_paint_tiles<T, nc_, sm ? kSmallX : kTileX, sm ? kSmallY : kTileY, sm ? kSmallZ : kTileZ, tb, decltype(D)::value, acc32>),
+            hipLaunchKernelGGL((k_paint_tiles<T, nc_, decltype(TX)::value, decltype(TY)::value, decltype(TZ)::value, tb, decltype(D)::value,
+                                              decltype(ACC32)::value != 0>),
                                dim3((unsigned)tg.ntiles), dim3(tb), 0, st, pos, pd, np, mass, (T)mscalar, m, mp, tg, offsets, sorted, hdr, out_scale, out,
                                nc_ == 1 ? vmax_out : nullptr);
         });
     };
-    auto sized = [&](auto NC, auto TB, auto ACC32) {
-        if (small) deposit(NC, std::integral_constant<int, 1>{}, TB, ACC32);
-        else deposit(NC, std::integral_constant<int, 0>{}, TB, ACC32);
-    };
-    using std::integral_constant;
     KTimer _t(nc == 1 ? "paint_deposit1" : "paint_deposit3", st);
-    if (nc == 1) {
-        sized(integral_constant<int, 1>{}, integral_constant<int, kPaint1Block>{}, integral_constant<int, 0>{});
-    } else if (sizeof(T) == 4 && wmesh) {
-        if constexpr (sizeof(T) == 4) sized(integral_constant<int, 3>{}, integral_constant<int, kAcc32Block>{}, integral_constant<int, 1>{});
+    constexpr Int<0> no{};
+    constexpr Int<1> c1{};
+    constexpr Int<3> c3{};
+    const bool acc32 = sizeof(T) == 4 && nc == 3 && wmesh;
+    auto small = [&](auto NC, auto ACC32) { deposit(NC, Int<kSmallX>{}, Int<kSmallY>{}, Int<kSmallZ>{}, Int<kSmallBlock>{}, ACC32); };
+    auto flat = [&](auto NC, auto TB) { deposit(NC, Int<kTileX>{}, Int<kTileY>{}, Int<kFlatZ>{}, TB, no); };
+    auto large = [&](auto NC, auto TB, auto ACC32) { deposit(NC, Int<kTileX>{}, Int<kTileY>{}, Int<kTileZ>{}, TB, ACC32); };
+    if (acc32) {
+        if constexpr (sizeof(T) == 4) {
+            if (pt.split == kSplitSmall) small(c3, c1);
+            else large(c3, Int<kAcc32Block>{}, c1);
+        }
+    } else if (pt.split == kSplitSmall) {
+        if (nc == 1) small(c1, no);
+        else small(c3, no);
+    } else if (pt.split == kSplitFlat) {
+        if (nc == 3) flat(c3, Int<kFlat3Block>{});
+        else if constexpr (sizeof(T) == 8) flat(c1, Int<kFlat1Block>{});
+    } else if (nc == 1) {
+        large(c1, Int<kPaint1Block>{}, no);
     } else {
-        sized(integral_constant<int, 3>{}, integral_constant<int, 1024>{}, integral_constant<int, 0>{});
+        large(c3, Int<1024>{}, no);
     }
     LDL_LAUNCH_CHECK();
     return LDL_OK;
@@ -408,7 +448,7 @@ static int paint_noalloc(const T* pos, const ldl_pos_desc* pdesc, int64_t np, co
     if (np < 0) return fail(LDL_EINVAL, "np must be >= 0");
     // the array holds whatever the previous call left: never skip clearing
     flags &= ~LDL_PAINT_WS_ZEROED;
-    const size_t need = flags & LDL_PAINT_FLOAT_ATOMIC ? 0 : paint_ws(m, 1, np, flags, false).total;  // (sorts without the stray lists)
+    const size_t need = flags & LDL_PAINT_FLOAT_ATOMIC ? 0 : paint_ws(m, 1, np, flags, paint_tiles(m, np, false).tg, false).total;  // (sorts without the stray lists)
     if (need > kNoAllocScratchBytes)
         return fail(LDL_EINVAL, "ldl_ppaint_noalloc: this paint needs " + std::to_string(need) + " bytes of scratch, the fixed array holds " +
                                     std::to_string(kNoAllocScratchBytes) + " (use ldl_ppaint with a workspace)");
