@@ -8,6 +8,7 @@
 #include <string>
 
 #include "../../include/ldl.h"
+#include "pow64.h"
 
 namespace ldl {
 
@@ -426,7 +427,7 @@ struct KTimer {
 // ----------------------------------------------------- elementwise math
 // Power, log and exp of positive arguments: the FP32 path uses the hardware
 // log2 / exp2 / reciprocal instructions (a few ulp), the FP64 path the
-// accurate library routines.
+// accurate library routines, and pow64.h's powers where these bound a pass.
 constexpr float kLn2f = 0.693147180559945309f;
 __device__ __forceinline__ float ppow(float x, float y) { return __builtin_amdgcn_exp2f(y * __builtin_amdgcn_logf(x)); }
 __device__ __forceinline__ double ppow(double x, double y) { return pow(x, y); }
@@ -445,6 +446,26 @@ __device__ __forceinline__ void pow_pair_log(double x, double a, double& p, doub
     ln = log(x);
     p = pow(x, a);
     p1 = pow(x, a - 1.0);
+}
+// The two above for the density's rows in the layer's z passes, which the FP64
+// library calls bound (256^3: r2c 132 -> 115 us, gamma adjoint 287 -> 144).
+// The pointwise loss kernels keep those: the registers of both branches cost
+// them more than they gain (107 -> 144 us where the power is not even taken).
+__device__ __forceinline__ float row_pow(float x, float y) { return ppow(x, y); }
+__device__ __forceinline__ double row_pow(double x, double y) {
+    const LogPair g = log_pair(x);
+    return pow_pair_ok(x, y * g.h) ? pow_from_log(g, y) : pow(x, y);
+}
+__device__ __forceinline__ void row_pow_pair_log(float x, float a, float& p, float& p1, float& ln) { pow_pair_log(x, a, p, p1, ln); }
+__device__ __forceinline__ void row_pow_pair_log(double x, double a, double& p, double& p1, double& ln) {
+    const LogPair g = log_pair(x);
+    if (pow_pair_ok(x, a * g.h) && pow_pair_ok(x, (a - 1.0) * g.h)) {
+        ln = g.h;
+        p = pow_from_log(g, a);
+        p1 = pow_from_log(g, a - 1.0);
+    } else {
+        pow_pair_log(x, a, p, p1, ln);
+    }
 }
 
 // Per-particle streams of the gathers (positions, cotangents): read or

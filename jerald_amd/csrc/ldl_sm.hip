@@ -57,7 +57,7 @@ template <typename T> struct KTabs {
 // with the terms its parameter gradients reuse: th, tl with
 // dG/dkh = G gkh th and dG/dkl = G gkl tl (sm: th = 1/k^2, tl = k^2; dm:
 // th = 1/|k|, tl = |k|; gkh, gkl from the host), and ln|k|.  FP32: hardware
-// reciprocal, square root, log2 and exp2; FP64: library routines.
+// reciprocal, square root, log2 and exp2; FP64: pow64.h and library routines.
 template <typename T> struct SmFilter {
     T kh, inv_kl, nu;  // sm: kh^2, 1/kl^2; dm: kh, 1/kl
     int dm;
@@ -75,8 +75,10 @@ template <typename T> struct SmFilter {
             }
             G = -__expf(-tl * inv_kl - kh * th) * pw;
         } else {
-            lnk = 0.5 * log(k2);
-            const double pw = nu == 0.0 ? 1.0 : pow(k2, 0.5 * nu);
+            const LogPair g = log_pair(k2);
+            const bool ok = pow_pair_ok(k2, 0.5 * nu * g.h);
+            lnk = 0.5 * (ok ? g.h : log(k2));
+            const double pw = nu == 0.0 ? 1.0 : ok ? pow_from_log(g, 0.5 * nu) : pow(k2, 0.5 * nu);
             tl = dm ? sqrt(k2) : k2;
             th = 1.0 / tl;
             G = -exp(-tl * inv_kl - kh * th) * pw;
@@ -261,7 +263,7 @@ template <typename T> struct PowRowLoad {  // (rho + 1e-8)^gamma, model.py:193
     T gamma;
     __device__ __forceinline__ c2<T> load2(int64_t row, int m) const {
         const c2<T> r = *reinterpret_cast<const c2<T>*>(rho + row * n2 + 2 * m);
-        return c2<T>{ppow(r.x + T(1e-8), gamma), ppow(r.y + T(1e-8), gamma)};
+        return c2<T>{row_pow(r.x + T(1e-8), gamma), row_pow(r.y + T(1e-8), gamma)};
     }
 };
 
@@ -333,8 +335,8 @@ template <typename T> struct GammaBwdStore {
         const c2<T> r = *reinterpret_cast<const c2<T>*>(rho + i);
         const T g0 = v.x * scale, g1 = v.y * scale;
         T p0, q0, l0, p1, q1, l1;
-        pow_pair_log(r.x + T(1e-8), gamma, p0, q0, l0);
-        pow_pair_log(r.y + T(1e-8), gamma, p1, q1, l1);
+        row_pow_pair_log(r.x + T(1e-8), gamma, p0, q0, l0);
+        row_pow_pair_log(r.y + T(1e-8), gamma, p1, q1, l1);
         acc[0] += (double)(g0 * p0) * (double)l0 + (double)(g1 * p1) * (double)l1;
         *reinterpret_cast<c2<T>*>(grho + i) = c2<T>{g0 * gamma * q0, g1 * gamma * q1};
     }
