@@ -323,10 +323,10 @@ __global__ void __launch_bounds__(1024) k_zpass_r2c_any(int64_t nrows, const c2<
     }
 }
 
-// block_sum for a runtime workgroup size (a multiple of 64, at most 1024).
+// block_sum for a runtime workgroup size (a multiple of 64, at most 1024);
+// red holds NR * 16 values.
 template <int NR>
-__device__ __forceinline__ void block_sum_any(double (&v)[NR]) {
-    __shared__ double red[NR * 16];
+__device__ __forceinline__ void block_sum_any(double (&v)[NR], double* red) {
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, nw = blockDim.x >> 6;
 #pragma unroll
     for (int r = 0; r < NR; r++) {
@@ -406,7 +406,8 @@ __global__ void __launch_bounds__(1024) k_zpass_c2r_any(int64_t nrows, const c2<
         else epi.store2(row0 + p, m, a[m * LS + p], acc);
     }
     if constexpr (NR > 0) {
-        block_sum_any<NR>(acc);
+        __shared__ double red[NR * 16];
+        block_sum_any<NR>(acc, red);
         if (threadIdx.x == 0) epi.reduce_out(blockIdx.x, acc);
     }
 }

@@ -49,6 +49,13 @@ template <typename T> struct KTabs {
         const T k2 = a * a + b * b + c * c;
         return k2 == T(0) ? T(1e-8) * T(1e-8) : k2;
     }
+    // The same with its roundings spelt out, for loops along x, where the
+    // compiler would hoist the other squares and fuse differently.
+    __device__ __forceinline__ T knorm2_fma(int64_t ix, int64_t iy, int64_t iz) const {
+        const T a = k[0][ix], b = k[1][iy], c = k[2][iz];
+        const T k2 = __builtin_elementwise_fma(c, c, __builtin_elementwise_fma(a, a, b * b));
+        return k2 == T(0) ? T(1e-8) * T(1e-8) : k2;
+    }
 };
 
 // Green's kernel of a layer, from k^2 (|k| = 1e-8 at k = 0):
@@ -642,9 +649,8 @@ k_x_realfilter(ColGeom g, const c2<T>* __restrict__ tw, c2<T>* __restrict__ io, 
 // iz >= nh are skipped), which do what the fused x kernels do between their
 // transforms.
 
-// PHI: out3 = P = cpot alpha G U [+ a G2 S2], the potential's spectrum; else
-// the three force spectra out3[d] = -i D_d P.
-template <typename T, bool HI, bool PHI>
+// The three force spectra out3[d] = -i D_d P, P = cpot alpha G U [+ a G2 S2].
+template <typename T, bool HI>
 __global__ void __launch_bounds__(256) k_sm_filter_fwd(const c2<T>* __restrict__ U, c2<T>* __restrict__ out3, int64_t hcells, int64_t n1,
                                                        int64_t nh, int64_t hp, KTabs<T> kt, SmFilter<T> fl, T a1e2, Src2<T> s2) {
     for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < hcells; i += (int64_t)gridDim.x * blockDim.x) {
@@ -659,20 +665,16 @@ __global__ void __launch_bounds__(256) k_sm_filter_fwd(const c2<T>* __restrict__
             const T G2 = s2.a * s2.fl.G(k2);
             p = c2<T>{p.x + G2 * sv.x, p.y + G2 * sv.y};
         }
-        if constexpr (PHI) {
-            out3[i] = p;
-        } else {
-            const T D[3] = {kt.D[0][ix], kt.D[1][iy], kt.D[2][iz]};
+        const T D[3] = {kt.D[0][ix], kt.D[1][iy], kt.D[2][iz]};
 #pragma unroll
-            for (int d = 0; d < 3; d++) out3[d * hcells + i] = c2<T>{D[d] * p.y, -D[d] * p.x};
-        }
+        for (int d = 0; d < 3; d++) out3[d * hcells + i] = c2<T>{D[d] * p.y, -D[d] * p.x};
     }
 }
 
-// Q = S3 (PHI: the divergence's spectrum), else sum_d i D_d S_d; FP64 partials (alpha, kh, kl, nu; HI also alpha2,
-// kh2, kl2, nu2, gamma2) per workgroup into part[NP * block + j]; out =
-// cpot alpha G Q (out may alias S3's first spectrum).
-template <typename T, bool HI, bool PHI>
+// Q = sum_d i D_d S_d; FP64 partials (alpha, kh, kl, nu; HI also alpha2, kh2,
+// kl2, nu2, gamma2) per workgroup into part[NP * block + j]; out = cpot alpha
+// G Q (out may alias S3's first spectrum).
+template <typename T, bool HI>
 __global__ void __launch_bounds__(256) k_sm_filter_bwd(const c2<T>* S3, const c2<T>* __restrict__ U, c2<T>* out, int64_t hcells, int64_t n1,
                                                        int64_t nh, int64_t hp, int64_t n2, int64_t zdbl, KTabs<T> kt, SmFilter<T> fl, T a1e2, double gkh,
                                                        double gkl, double cpot, double alpha, int alpha_rule, Src2<T> s2,
@@ -684,15 +686,11 @@ __global__ void __launch_bounds__(256) k_sm_filter_bwd(const c2<T>* S3, const c2
         const int64_t iz = i % hp, iy = (i / hp) % n1, ix = i / (hp * n1);
         if (iz >= nh) continue;
         c2<T> q = c2<T>{T(0), T(0)};
-        if constexpr (PHI) {
-            q = S3[i];
-        } else {
-            const T D[3] = {kt.D[0][ix], kt.D[1][iy], kt.D[2][iz]};
+        const T D[3] = {kt.D[0][ix], kt.D[1][iy], kt.D[2][iz]};
 #pragma unroll
-            for (int d = 0; d < 3; d++) {
-                const c2<T> v = S3[d * hcells + i];
-                q = c2<T>{q.x - D[d] * v.y, q.y + D[d] * v.x};  // += i D v
-            }
+        for (int d = 0; d < 3; d++) {
+            const c2<T> v = S3[d * hcells + i];
+            q = c2<T>{q.x - D[d] * v.y, q.y + D[d] * v.x};  // += i D v
         }
         const T G = xbwd_cell<T, HI>(fl, s2, kt.knorm2(ix, iy, iz), q, U[i], i, xbwd_weights(iz, n2, zdbl, alpha_rule), cpot, apot, gkh,
                                      gkl, acc);
@@ -701,6 +699,225 @@ __global__ void __launch_bounds__(256) k_sm_filter_bwd(const c2<T>* S3, const c2
     block_sum<NP, 256>(acc);
     if (threadIdx.x == 0)
         for (int j = 0; j < NP; j++) part[blockIdx.x * NP + j] = acc[j];
+}
+
+// The fused x passes for x lengths with factors 3 and 5.  FP64 (PHI) carries
+// the potential's one spectrum, as k_sm_x_fwd and k_sm_x_bwd do; FP32 the three
+// force spectra, hc apart, whose bits the separate passes above also give.
+// They are bound by the memory they move: one read of the tile and one write
+// per spectrum, where separate transforms and filter passes read and wrote
+// each spectrum twice more (384^3 FP32 forward 720 -> 423 us).  A thread holds elements q + s nq, s < 16,
+// of column p between transforms.
+template <typename T, int P, bool HI>
+__global__ void __launch_bounds__(1024) k_sm_x_any_fwd(ColGeom g, const c2<T>* __restrict__ tw, AnyPlan pl, c2<T>* __restrict__ U, c2<T>* __restrict__ out,
+                                                       int64_t hc, KTabs<T> kt, SmFilter<T> fl, T a1e2, T invM, Src2<T> s2) {
+    using C = c2<T>;
+    extern __shared__ __align__(16) unsigned char any_smem[];
+    constexpr bool PHI = sizeof(T) == 8;
+    constexpr int LS = P + 1, NV = 16;
+    const int n = pl.n, nq = (int)blockDim.x / P;
+    C* a = reinterpret_cast<C*>(any_smem);
+    C* twl = a + n * LS;
+    const int64_t tile = xcd_tile(blockIdx.x, gridDim.x);
+    const int64_t plane = tile / g.tiles_per_plane;
+    const int64_t col0 = (tile - plane * g.tiles_per_plane) * P;
+    const int64_t base = plane * g.plane_stride + col0;
+    const int pv = (int)((g.ncols - col0) < P ? (g.ncols - col0) : P);
+    const int p = threadIdx.x % P, q = threadIdx.x / P, pc = p < pv ? p : pv - 1;
+    for (int i = threadIdx.x; i < n; i += blockDim.x) twl[i] = tw[i];
+    C v[NV];  // all of a thread's loads before the first LDS write
+#pragma unroll
+    for (int s = 0; s < NV; s++) {
+        const int nn = q + s * nq;
+        if (nn < n) v[s] = U[base + nn * g.es + pc];
+    }
+#pragma unroll
+    for (int s = 0; s < NV; s++) {
+        const int nn = q + s * nq;
+        if (nn < n) a[nn * LS + p] = p < pv ? v[s] : C{T(0), T(0)};
+    }
+    __syncthreads();
+    any_fft<T, -1, P>(a, twl, 1, pl);
+    auto cell = [&](int nn) {
+        C u = a[nn * LS + p];
+        u = C{u.x * invM, u.y * invM};
+        const int64_t i = base + nn * g.es + p;
+        U[i] = u;
+        const T k2 = kt.knorm2_fma(nn, plane, col0 + p);
+        const T G = fl.G(k2);
+        C r = C{u.x * a1e2 * G, u.y * a1e2 * G};
+        if constexpr (HI) {
+            const C sv = s2.S[i];
+            const T G2 = s2.a * s2.fl.G(k2);
+            r = C{r.x + G2 * sv.x, r.y + G2 * sv.y};
+        }
+        return r;
+    };
+    if constexpr (PHI) {
+        if (p < pv)
+            for (int nn = q; nn < n; nn += nq) a[nn * LS + p] = cell(nn);
+        __syncthreads();
+        any_fft<T, +1, P>(a, twl, 1, pl);
+        if (p < pv)
+            for (int nn = q; nn < n; nn += nq) out[base + nn * g.es + p] = a[nn * LS + p];
+    } else {
+#pragma unroll
+        for (int s = 0; s < NV; s++) {
+            const int nn = q + s * nq;
+            v[s] = C{T(0), T(0)};
+            if (nn < n && p < pv) v[s] = cell(nn);
+        }
+        const T D1 = kt.D[1][plane], D2 = kt.D[2][col0 + pc];
+#pragma unroll 1
+        for (int d = 0; d < 3; d++) {  // each thread rewrites its own elements only
+#pragma unroll
+            for (int s = 0; s < NV; s++) {
+                const int nn = q + s * nq;
+                if (nn < n) {
+                    const T D = d == 0 ? kt.D[0][nn] : d == 1 ? D1 : D2;
+                    a[nn * LS + p] = C{D * v[s].y, -D * v[s].x};
+                }
+            }
+            __syncthreads();
+            any_fft<T, +1, P>(a, twl, 1, pl);
+            if (p < pv)
+                for (int nn = q; nn < n; nn += nq) out[d * hc + base + nn * g.es + p] = a[nn * LS + p];
+        }
+    }
+}
+
+template <typename T, int P, bool HI>
+__global__ void __launch_bounds__(1024) k_sm_x_any_bwd(ColGeom g, const c2<T>* S3, const c2<T>* __restrict__ tw, AnyPlan pl, const c2<T>* __restrict__ U,
+                                                       c2<T>* out, int64_t hc, int64_t n2, int64_t zdbl, KTabs<T> kt, SmFilter<T> fl, T a1e2, double gkh,
+                                                       double gkl, double cpot, double alpha, int alpha_rule, Src2<T> s2, double* __restrict__ part) {
+    using C = c2<T>;
+    extern __shared__ __align__(16) unsigned char any_smem[];
+    constexpr bool PHI = sizeof(T) == 8;
+    constexpr int LS = P + 1, NV = 16;
+    const int n = pl.n, nq = (int)blockDim.x / P;
+    C* a = reinterpret_cast<C*>(any_smem);
+    C* twl = a + n * LS;
+    const int64_t tile = xcd_tile(blockIdx.x, gridDim.x);
+    const int64_t plane = tile / g.tiles_per_plane;
+    const int64_t col0 = (tile - plane * g.tiles_per_plane) * P;
+    const int64_t base = plane * g.plane_stride + col0;
+    const int pv = (int)((g.ncols - col0) < P ? (g.ncols - col0) : P);
+    const int p = threadIdx.x % P, q = threadIdx.x / P, pc = p < pv ? p : pv - 1;
+    for (int i = threadIdx.x; i < n; i += blockDim.x) twl[i] = tw[i];
+    auto transform = [&](const C* S) {
+        C v[NV];  // all of a thread's loads before the first LDS write
+#pragma unroll
+        for (int s = 0; s < NV; s++) {
+            const int nn = q + s * nq;
+            if (nn < n) v[s] = S[base + nn * g.es + pc];
+        }
+#pragma unroll
+        for (int s = 0; s < NV; s++) {
+            const int nn = q + s * nq;
+            if (nn < n) a[nn * LS + p] = p < pv ? v[s] : C{T(0), T(0)};
+        }
+        __syncthreads();
+        any_fft<T, -1, P>(a, twl, 1, pl);
+    };
+    if constexpr (PHI) {
+        transform(S3);
+    } else {
+        C Q[NV];
+#pragma unroll
+        for (int s = 0; s < NV; s++) Q[s] = C{T(0), T(0)};
+        const T D1 = kt.D[1][plane], D2 = kt.D[2][col0 + pc];
+#pragma unroll 1
+        for (int d = 0; d < 3; d++) {
+            transform(S3 + d * hc);
+#pragma unroll
+            for (int s = 0; s < NV; s++) {
+                const int nn = q + s * nq;
+                if (nn < n) {
+                    const T D = d == 0 ? kt.D[0][nn] : d == 1 ? D1 : D2;
+                    const C w = a[nn * LS + p];
+                    Q[s] = C{Q[s].x - D * w.y, Q[s].y + D * w.x};  // += i D v
+                }
+            }
+        }
+#pragma unroll
+        for (int s = 0; s < NV; s++) {
+            const int nn = q + s * nq;
+            if (nn < n) a[nn * LS + p] = Q[s];
+        }
+    }
+    constexpr int NP = HI ? 9 : 4;
+    double acc[NP] = {};
+    const double apot = cpot * alpha;
+    if (p < pv) {  // each thread rewrites its own elements only
+        const int64_t kz = col0 + p;
+        for (int nn = q; nn < n; nn += nq) {
+            const C w = a[nn * LS + p];
+            const int64_t i = base + nn * g.es + p;
+            const T G = xbwd_cell<T, HI>(fl, s2, kt.knorm2_fma(nn, plane, kz), w, U[i], i, xbwd_weights(kz, n2, zdbl, alpha_rule), cpot, apot, gkh, gkl, acc);
+            a[nn * LS + p] = C{a1e2 * G * w.x, a1e2 * G * w.y};
+        }
+    }
+    __syncthreads();
+    any_fft<T, +1, P>(a, twl, 1, pl);
+    if (p < pv)
+        for (int nn = q; nn < n; nn += nq) out[base + nn * g.es + p] = a[nn * LS + p];
+    __shared__ double red[NP * 16];
+    block_sum_any<NP>(acc, red);
+    if (threadIdx.x == 0) {
+#pragma unroll
+        for (int j = 0; j < NP; j++) part[blockIdx.x * NP + j] = acc[j];
+    }
+}
+
+// Whether the layer's x passes run fused with the power-of-two kernels: every
+// axis a power of two, or the x axis in FP64 (FP32 keeps the bits that the
+// separate passes have on such meshes).
+template <typename T> static bool x_pow2(const Mesh& m) { return fft_mesh_pow2(m) || (sizeof(T) == 8 && pow2_len(m.n0, 1024)); }
+
+// Launch shape of a fused any-length x pass.  Its chains of up to four
+// transforms leave it bound by latency more than the plain passes, so of 16 and
+// 8 pencils (FP64: 8 and 4) it takes those that keep more wavefronts on a CU
+// (at most 16 at its 128 VGPRs), and with as many the FP32 pass the 8, the FP64
+// pass the 8.  A workgroup has at least 128 threads (FP64: 256) where the
+// transform has butterflies for them, 512 in a pass of too few pencils to fill
+// the chip.  Forward and backward, us, against the plain passes' shapes: 384^3
+// FP32 429 and 759 -> 423 and 715, FP64 536 and 749 -> 440 and 617; 320^3 FP32
+// 300 and 571 -> 245 and 428; 240^3 FP64 145 and 199 -> 110 and 160; 100^3 FP32
+// 24 and 35 -> 23 and 32, FP64 29 and 34 -> 21 and 25.
+template <typename T>
+static AnyShape x_any_shape(AnyPlan* pl, int64_t pencils) {
+    constexpr int PM = sizeof(T) == 4 ? 16 : 8, least = sizeof(T) == 4 ? 128 : 256;
+    const int n = pl->n, few = pl->tpp;
+    int most = few;
+    for (int i = 0; i < pl->ngrp; i++) most = std::max(most, pl->g[i].nbg);
+    auto shape = [&](int P, int threads) {
+        pl->tpp = std::max(few, std::min(most, threads / P));
+        return AnyShape{P, (P * pl->tpp + 63) / 64 * 64, ((size_t)n * (P + 1) + n) * sizeof(c2<T>)};
+    };
+    auto waves = [&](const AnyShape& s) {
+        return s.th > 1024 || s.lds > 158 * 1024 ? 0 : std::min<int>(16, (int)((size_t)160 * 1024 / (s.lds + 1280)) * (s.th / 64));
+    };
+    if (pencils <= 1024 * PM / 2) return shape(PM / 2, 512);
+    const int wm = waves(shape(PM, least)), wh = waves(shape(PM / 2, least));
+    return shape(wm > wh || (sizeof(T) == 8 && wm == wh) ? PM : PM / 2, least);
+}
+
+// Geometry, plan and shape of a fused any-length x pass: f(P, geometry, plan, twiddles, shape).
+template <typename T, class F>
+static int x_any(const Mesh& m, int64_t nh, int64_t hp, F&& f) {
+    AnyPlan pl;
+    if (!any_plan(m.n0, &pl)) return fail(LDL_EUNSUPPORTED, "FFT length must have no prime factor other than 2, 3 and 5");
+    const c2<T>* twn;
+    const int rc = twiddles_n<T>((int)m.n0, &twn);
+    if (rc) return rc;
+    const AnyShape sh = x_any_shape<T>(&pl, m.n1 * nh);
+    with_any_p<T>(sh, [&](auto PC) {
+        constexpr int P = decltype(PC)::value;
+        ColGeom g{m.n1, nh, hp, m.n1 * hp, (nh + P - 1) / P, 0};
+        g.ntiles = g.tiles_per_plane * m.n1;
+        f(PC, g, pl, twn, sh);
+    });
+    return LDL_OK;
 }
 
 // S *= scale * W(k) (the weights of k_x_realfilter, k = 0 bin set to 0)
@@ -1392,7 +1609,7 @@ static int sm_layer_fwd(int kind, const T* pos, const ldl_pos_desc* pdesc, int64
     // 3. x pass + filter + inverse x pass (and the x difference)
     const SmFilter<T> fl = layer_filter<T>(prm, kind == kKindDm);
     const T a1e2 = (T)((hi ? 1e-3 : 1e-2) * prm[0]);
-    if (fft_mesh_pow2(m)) {
+    if (x_pow2<T>(m)) {
         dispatch_n(m.n0, [&](auto N) {
             constexpr int NN = decltype(N)::value;
             ColGeom g = col_geom<T, NN>(m.n1, nh, hp, m.n1 * hp);
@@ -1405,15 +1622,26 @@ static int sm_layer_fwd(int kind, const T* pos, const ldl_pos_desc* pdesc, int64
                 hipLaunchKernelGGL((k_sm_x_fwd<T, NN, false>), dim3((unsigned)g.ntiles), dim3(XTH), 0, st, g, tw, U, P.spec3,
                                    kt, fl, a1e2, invM, s2);
         });
-    } else {
+    } else if (!pow2_len(m.n0, 1024)) {
+        rc = x_any<T>(m, nh, hp, [&](auto PC, const ColGeom& g, const AnyPlan& pl, const c2<T>* twn, const AnyShape& sh) {
+            constexpr int XP = decltype(PC)::value;
+            auto run = [&](auto* kernel) {
+                allow_lds(kernel, sh.lds);
+                KTimer _t("sm_x_fwd", st);
+                hipLaunchKernelGGL(kernel, dim3((unsigned)g.ntiles), dim3(sh.th), sh.lds, st, g, twn, pl, U, P.spec3, hc, kt, fl, a1e2, invM, s2);
+            };
+            if (hi) run(&k_sm_x_any_fwd<T, XP, true>);
+            else run(&k_sm_x_any_fwd<T, XP, false>);
+        });
+        if (rc) return rc;
+    } else if constexpr (sizeof(T) == 4) {
         if ((rc = colpass<T, -1>(m.n0, m.n1, nh, hp, m.n1 * hp, tw, PlainColOp<T>{U, U, invM}, st))) return rc;
         const unsigned gf = grid_for(hc, 256, 1 << 16);
-        constexpr bool PHI = sizeof(T) == 8;
         if (hi)
-            hipLaunchKernelGGL((k_sm_filter_fwd<T, true, PHI>), dim3(gf), dim3(256), 0, st, U, P.spec3, hc, m.n1, nh, hp, kt, fl, a1e2, s2);
+            hipLaunchKernelGGL((k_sm_filter_fwd<T, true>), dim3(gf), dim3(256), 0, st, U, P.spec3, hc, m.n1, nh, hp, kt, fl, a1e2, s2);
         else
-            hipLaunchKernelGGL((k_sm_filter_fwd<T, false, PHI>), dim3(gf), dim3(256), 0, st, U, P.spec3, hc, m.n1, nh, hp, kt, fl, a1e2, s2);
-        for (int d = 0; d < (PHI ? 1 : 3); d++)
+            hipLaunchKernelGGL((k_sm_filter_fwd<T, false>), dim3(gf), dim3(256), 0, st, U, P.spec3, hc, m.n1, nh, hp, kt, fl, a1e2, s2);
+        for (int d = 0; d < 3; d++)
             if ((rc = colpass<T, +1>(m.n0, m.n1, nh, hp, m.n1 * hp, tw, PlainColOp<T>{P.spec3 + d * hc, P.spec3 + d * hc, T(1)}, st))) return rc;
     }
     // 4. inverse y passes (3 force spectra as 3*N0 planes) and z c2r into F
@@ -1511,7 +1739,7 @@ static int sm_layer_bwd(int kind, const T* pos, const ldl_pos_desc* pdesc, int64
     const int64_t zdbl = std::min<int64_t>(m.n1 / 2, nh);  // end of c2f's doubled z bins (reference rule)
     c2<T>* S = P.spec3;  // result reuses the first spectrum (read before written)
     int64_t ntx = 0;
-    if (fft_mesh_pow2(m)) {
+    if (x_pow2<T>(m)) {
         dispatch_n(m.n0, [&](auto N) {
             constexpr int NN = decltype(N)::value;
             ColGeom g = col_geom<T, NN, xbwd_pencils<T, NN>()>(m.n1, nh, hp, m.n1 * hp);
@@ -1525,18 +1753,31 @@ static int sm_layer_bwd(int kind, const T* pos, const ldl_pos_desc* pdesc, int64
                 hipLaunchKernelGGL((k_sm_x_bwd<T, NN, false>), dim3((unsigned)g.ntiles), dim3(XTH), 0, st, g, P.spec3, tw, U,
                                    S, m.n2, zdbl, kt, fl, a1e2, gkh, gkl, cpot, prm[0], (int)alpha_rule, s2, P.part);
         });
-    } else {
-        constexpr bool PHI = sizeof(T) == 8;
-        for (int d = 0; d < (PHI ? 1 : 3); d++)
+    } else if (!pow2_len(m.n0, 1024)) {
+        rc = x_any<T>(m, nh, hp, [&](auto PC, const ColGeom& g, const AnyPlan& pl, const c2<T>* twn, const AnyShape& sh) {
+            constexpr int XP = decltype(PC)::value;
+            ntx = g.ntiles;
+            auto run = [&](auto* kernel) {
+                allow_lds(kernel, sh.lds);
+                KTimer _t("sm_x_bwd", st);
+                hipLaunchKernelGGL(kernel, dim3((unsigned)g.ntiles), dim3(sh.th), sh.lds, st, g, (const c2<T>*)P.spec3, twn, pl, U, S, hc, m.n2, zdbl, kt, fl,
+                                   a1e2, gkh, gkl, cpot, prm[0], (int)alpha_rule, s2, P.part);
+            };
+            if (hi) run(&k_sm_x_any_bwd<T, XP, true>);
+            else run(&k_sm_x_any_bwd<T, XP, false>);
+        });
+        if (rc) return rc;
+    } else if constexpr (sizeof(T) == 4) {
+        for (int d = 0; d < 3; d++)
             if ((rc = colpass<T, -1>(m.n0, m.n1, nh, hp, m.n1 * hp, tw, PlainColOp<T>{P.spec3 + d * hc, P.spec3 + d * hc, T(1)}, st))) return rc;
         const unsigned gf = grid_for(hc, 256, 4096);
         ntx = gf;
         if (hi)
-            hipLaunchKernelGGL((k_sm_filter_bwd<T, true, PHI>), dim3(gf), dim3(256), 0, st, P.spec3, U, S, hc, m.n1, nh, hp, m.n2, zdbl, kt, fl, a1e2,
-                               gkh, gkl, cpot, prm[0], (int)alpha_rule, s2, P.part);
+            hipLaunchKernelGGL((k_sm_filter_bwd<T, true>), dim3(gf), dim3(256), 0, st, P.spec3, U, S, hc, m.n1, nh, hp, m.n2, zdbl, kt, fl, a1e2, gkh, gkl,
+                               cpot, prm[0], (int)alpha_rule, s2, P.part);
         else
-            hipLaunchKernelGGL((k_sm_filter_bwd<T, false, PHI>), dim3(gf), dim3(256), 0, st, P.spec3, U, S, hc, m.n1, nh, hp, m.n2, zdbl, kt, fl, a1e2,
-                               gkh, gkl, cpot, prm[0], (int)alpha_rule, s2, P.part);
+            hipLaunchKernelGGL((k_sm_filter_bwd<T, false>), dim3(gf), dim3(256), 0, st, P.spec3, U, S, hc, m.n1, nh, hp, m.n2, zdbl, kt, fl, a1e2, gkh, gkl,
+                               cpot, prm[0], (int)alpha_rule, s2, P.part);
         if ((rc = colpass<T, +1>(m.n0, m.n1, nh, hp, m.n1 * hp, tw, PlainColOp<T>{S, S, T(1)}, st))) return rc;
     }
     // partial columns -> parameter slots: alpha, kh, kl, nu (HI: then alpha2,
