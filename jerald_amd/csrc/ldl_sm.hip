@@ -643,8 +643,10 @@ k_x_realfilter(ColGeom g, const c2<T>* __restrict__ tw, c2<T>* __restrict__ io, 
 }
 
 // ------------------------------------ spectral kernels of the any-length path
-// Meshes whose axes are not all powers of two run the x passes unfused: plain
-// column passes around these elementwise kernels over the half spectrum
+// FP32 layers whose x axis is a power of two and another axis is not run plain
+// column passes around the next two kernels; the loss smoothing of meshes whose
+// axes are not all powers of two runs them around k_realfilter_mult.  All go
+// over the half spectrum
 // (index i -> (ix, iy, iz) with iz fastest, rows of pitch hp; the pad columns
 // iz >= nh are skipped), which do what the fused x kernels do between their
 // transforms.
