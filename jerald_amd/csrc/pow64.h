@@ -4,7 +4,9 @@
 // instructions, not by memory, with library calls (each pow forms its own
 // extended logarithm; the gamma adjoint took two of them and a log).  Here
 // ln x = h + l is formed once to about 2^-60 and each power is one
-// exponential of a (h + l), within 0.54 ulp where a |ln x| <= 700.  Arguments
+// exponential of a (h + l), within 0.58 ulp where a |ln x| <= 700 (the library pow:
+// 1.3 ulp over the same arguments).  256^3: gamma adjoint 287 -> 144 us, density
+// spectrum 132 -> 115.  Arguments
 // beyond that (zero, negative, subnormal, infinite and NaN bases, powers near
 // overflow or underflow) take the library's pow.
 //
