@@ -643,7 +643,7 @@ k_x_realfilter(ColGeom g, const c2<T>* __restrict__ tw, c2<T>* __restrict__ io, 
 }
 
 // ------------------------------------ spectral kernels of the any-length path
-// FP32 layers whose x axis is a power of two and another axis is not run plain
+// Layers whose x axis is a power of two and another axis is not run plain
 // column passes around the next two kernels; the loss smoothing of meshes whose
 // axes are not all powers of two runs them around k_realfilter_mult.  All go
 // over the half spectrum
@@ -703,19 +703,22 @@ __global__ void __launch_bounds__(256) k_sm_filter_bwd(const c2<T>* S3, const c2
         for (int j = 0; j < NP; j++) part[blockIdx.x * NP + j] = acc[j];
 }
 
-// The fused x passes for x lengths with factors 3 and 5.  FP64 (PHI) carries
-// the potential's one spectrum, as k_sm_x_fwd and k_sm_x_bwd do; FP32 the three
-// force spectra, hc apart, whose bits the separate passes above also give.
-// They are bound by the memory they move: one read of the tile and one write
-// per spectrum, where separate transforms and filter passes read and wrote
-// each spectrum twice more (384^3 FP32 forward 720 -> 423 us).  A thread holds elements q + s nq, s < 16,
-// of column p between transforms.
+// The fused x passes for x lengths with factors 3 and 5.  They carry the three
+// force spectra, hc apart, with the bits that the separate passes above also
+// give.  They are bound by the memory they move: one read of the tile and one
+// write per spectrum, where separate transforms and filter passes read and
+// wrote each spectrum twice more (384^3 FP32 forward 720 -> 423 us; FP64
+// one dm layer, loss and gradient 21.5 -> 20.6 ms).  A
+// thread holds elements q + s nq, s < 16, of column p between transforms:
+// in FP64 64 VGPRs beside the transform's 64, so it gets 256 and at most 512
+// threads share a workgroup.
+template <typename T> constexpr int x_any_most() { return sizeof(T) == 4 ? 1024 : 512; }
+
 template <typename T, int P, bool HI>
-__global__ void __launch_bounds__(1024) k_sm_x_any_fwd(ColGeom g, const c2<T>* __restrict__ tw, AnyPlan pl, c2<T>* __restrict__ U, c2<T>* __restrict__ out,
+__global__ void __launch_bounds__(x_any_most<T>()) k_sm_x_any_fwd(ColGeom g, const c2<T>* __restrict__ tw, AnyPlan pl, c2<T>* __restrict__ U, c2<T>* __restrict__ out,
                                                        int64_t hc, KTabs<T> kt, SmFilter<T> fl, T a1e2, T invM, Src2<T> s2) {
     using C = c2<T>;
     extern __shared__ __align__(16) unsigned char any_smem[];
-    constexpr bool PHI = sizeof(T) == 8;
     constexpr int LS = P + 1, NV = 16;
     const int n = pl.n, nq = (int)blockDim.x / P;
     C* a = reinterpret_cast<C*>(any_smem);
@@ -755,46 +758,36 @@ __global__ void __launch_bounds__(1024) k_sm_x_any_fwd(ColGeom g, const c2<T>* _
         }
         return r;
     };
-    if constexpr (PHI) {
-        if (p < pv)
-            for (int nn = q; nn < n; nn += nq) a[nn * LS + p] = cell(nn);
-        __syncthreads();
-        any_fft<T, +1, P>(a, twl, 1, pl);
-        if (p < pv)
-            for (int nn = q; nn < n; nn += nq) out[base + nn * g.es + p] = a[nn * LS + p];
-    } else {
+#pragma unroll
+    for (int s = 0; s < NV; s++) {
+        const int nn = q + s * nq;
+        v[s] = C{T(0), T(0)};
+        if (nn < n && p < pv) v[s] = cell(nn);
+    }
+    const T D1 = kt.D[1][plane], D2 = kt.D[2][col0 + pc];
+#pragma unroll 1
+    for (int d = 0; d < 3; d++) {  // each thread rewrites its own elements only
 #pragma unroll
         for (int s = 0; s < NV; s++) {
             const int nn = q + s * nq;
-            v[s] = C{T(0), T(0)};
-            if (nn < n && p < pv) v[s] = cell(nn);
-        }
-        const T D1 = kt.D[1][plane], D2 = kt.D[2][col0 + pc];
-#pragma unroll 1
-        for (int d = 0; d < 3; d++) {  // each thread rewrites its own elements only
-#pragma unroll
-            for (int s = 0; s < NV; s++) {
-                const int nn = q + s * nq;
-                if (nn < n) {
-                    const T D = d == 0 ? kt.D[0][nn] : d == 1 ? D1 : D2;
-                    a[nn * LS + p] = C{D * v[s].y, -D * v[s].x};
-                }
+            if (nn < n) {
+                const T D = d == 0 ? kt.D[0][nn] : d == 1 ? D1 : D2;
+                a[nn * LS + p] = C{D * v[s].y, -D * v[s].x};
             }
-            __syncthreads();
-            any_fft<T, +1, P>(a, twl, 1, pl);
-            if (p < pv)
-                for (int nn = q; nn < n; nn += nq) out[d * hc + base + nn * g.es + p] = a[nn * LS + p];
         }
+        __syncthreads();
+        any_fft<T, +1, P>(a, twl, 1, pl);
+        if (p < pv)
+            for (int nn = q; nn < n; nn += nq) out[d * hc + base + nn * g.es + p] = a[nn * LS + p];
     }
 }
 
 template <typename T, int P, bool HI>
-__global__ void __launch_bounds__(1024) k_sm_x_any_bwd(ColGeom g, const c2<T>* S3, const c2<T>* __restrict__ tw, AnyPlan pl, const c2<T>* __restrict__ U,
+__global__ void __launch_bounds__(x_any_most<T>()) k_sm_x_any_bwd(ColGeom g, const c2<T>* S3, const c2<T>* __restrict__ tw, AnyPlan pl, const c2<T>* __restrict__ U,
                                                        c2<T>* out, int64_t hc, int64_t n2, int64_t zdbl, KTabs<T> kt, SmFilter<T> fl, T a1e2, double gkh,
                                                        double gkl, double cpot, double alpha, int alpha_rule, Src2<T> s2, double* __restrict__ part) {
     using C = c2<T>;
     extern __shared__ __align__(16) unsigned char any_smem[];
-    constexpr bool PHI = sizeof(T) == 8;
     constexpr int LS = P + 1, NV = 16;
     const int n = pl.n, nq = (int)blockDim.x / P;
     C* a = reinterpret_cast<C*>(any_smem);
@@ -821,31 +814,27 @@ __global__ void __launch_bounds__(1024) k_sm_x_any_bwd(ColGeom g, const c2<T>* S
         __syncthreads();
         any_fft<T, -1, P>(a, twl, 1, pl);
     };
-    if constexpr (PHI) {
-        transform(S3);
-    } else {
-        C Q[NV];
+    C Q[NV];
 #pragma unroll
-        for (int s = 0; s < NV; s++) Q[s] = C{T(0), T(0)};
-        const T D1 = kt.D[1][plane], D2 = kt.D[2][col0 + pc];
+    for (int s = 0; s < NV; s++) Q[s] = C{T(0), T(0)};
+    const T D1 = kt.D[1][plane], D2 = kt.D[2][col0 + pc];
 #pragma unroll 1
-        for (int d = 0; d < 3; d++) {
-            transform(S3 + d * hc);
-#pragma unroll
-            for (int s = 0; s < NV; s++) {
-                const int nn = q + s * nq;
-                if (nn < n) {
-                    const T D = d == 0 ? kt.D[0][nn] : d == 1 ? D1 : D2;
-                    const C w = a[nn * LS + p];
-                    Q[s] = C{Q[s].x - D * w.y, Q[s].y + D * w.x};  // += i D v
-                }
-            }
-        }
+    for (int d = 0; d < 3; d++) {
+        transform(S3 + d * hc);
 #pragma unroll
         for (int s = 0; s < NV; s++) {
             const int nn = q + s * nq;
-            if (nn < n) a[nn * LS + p] = Q[s];
+            if (nn < n) {
+                const T D = d == 0 ? kt.D[0][nn] : d == 1 ? D1 : D2;
+                const C w = a[nn * LS + p];
+                Q[s] = C{Q[s].x - D * w.y, Q[s].y + D * w.x};  // += i D v
+            }
         }
+    }
+#pragma unroll
+    for (int s = 0; s < NV; s++) {
+        const int nn = q + s * nq;
+        if (nn < n) a[nn * LS + p] = Q[s];
     }
     constexpr int NP = HI ? 9 : 4;
     double acc[NP] = {};
@@ -871,24 +860,21 @@ __global__ void __launch_bounds__(1024) k_sm_x_any_bwd(ColGeom g, const c2<T>* S
     }
 }
 
-// Whether the layer's x passes run fused with the power-of-two kernels: every
-// axis a power of two, or the x axis in FP64 (FP32 keeps the bits that the
-// separate passes have on such meshes).
-template <typename T> static bool x_pow2(const Mesh& m) { return fft_mesh_pow2(m) || (sizeof(T) == 8 && pow2_len(m.n0, 1024)); }
-
-// Launch shape of a fused any-length x pass.  Its chains of up to four
-// transforms leave it bound by latency more than the plain passes, so of 16 and
-// 8 pencils (FP64: 8 and 4) it takes those that keep more wavefronts on a CU
-// (at most 16 at its 128 VGPRs), and with as many the FP32 pass the 8, the FP64
-// pass the 8.  A workgroup has at least 128 threads (FP64: 256) where the
-// transform has butterflies for them, 512 in a pass of too few pencils to fill
-// the chip.  Forward and backward, us, against the plain passes' shapes: 384^3
-// FP32 429 and 759 -> 423 and 715, FP64 536 and 749 -> 440 and 617; 320^3 FP32
-// 300 and 571 -> 245 and 428; 240^3 FP64 145 and 199 -> 110 and 160; 100^3 FP32
-// 24 and 35 -> 23 and 32, FP64 29 and 34 -> 21 and 25.
+// Launch shape of a fused any-length x pass.  Its chains of four transforms
+// leave it bound by latency more than the plain passes, so of 16 and 8 pencils
+// (FP64: 8 and 4) it takes those that keep more wavefronts on a CU (at most 16
+// at FP32's 128 VGPRs, 8 at FP64's 256, there in whole workgroups), and with as
+// many the 8.  A workgroup has at least 128 threads where the transform has
+// butterflies for them, 512 in a pass of too few pencils to fill the chip.
+// Forward and backward, us, FP32 against the plain passes' shapes: 384^3 429
+// and 759 -> 423 and 715; 320^3 300 and 571 -> 245 and 428; 100^3 24 and 35 ->
+// 23 and 32.  FP64, 8 pencils x 128 threads, 8 x 256 and 4 x 128: 100^3 36 and
+// 37, 42 and 45, 42 and 45; 240^3 222 and 236, 271 and 298, 270 and 288; 320^3
+// 626 and 673 (3 wavefronts a workgroup, 6 on a CU), 558 and 608, 543 and 580;
+// 384^3 907 and 987, 913 and 992, 922 and 940.
 template <typename T>
 static AnyShape x_any_shape(AnyPlan* pl, int64_t pencils) {
-    constexpr int PM = sizeof(T) == 4 ? 16 : 8, least = sizeof(T) == 4 ? 128 : 256;
+    constexpr int PM = sizeof(T) == 4 ? 16 : 8, least = 128, cap = x_any_most<T>() / 64;
     const int n = pl->n, few = pl->tpp;
     int most = few;
     for (int i = 0; i < pl->ngrp; i++) most = std::max(most, pl->g[i].nbg);
@@ -897,7 +883,9 @@ static AnyShape x_any_shape(AnyPlan* pl, int64_t pencils) {
         return AnyShape{P, (P * pl->tpp + 63) / 64 * 64, ((size_t)n * (P + 1) + n) * sizeof(c2<T>)};
     };
     auto waves = [&](const AnyShape& s) {
-        return s.th > 1024 || s.lds > 158 * 1024 ? 0 : std::min<int>(16, (int)((size_t)160 * 1024 / (s.lds + 1280)) * (s.th / 64));
+        const int w = s.th / 64, groups = (int)((size_t)160 * 1024 / (s.lds + 1280));
+        if (w > cap || s.lds > 158 * 1024) return 0;
+        return sizeof(T) == 4 ? std::min(cap, groups * w) : std::min(groups, cap / w) * w;
     };
     if (pencils <= 1024 * PM / 2) return shape(PM / 2, 512);
     const int wm = waves(shape(PM, least)), wh = waves(shape(PM / 2, least));
@@ -1553,15 +1541,6 @@ static int check_prm(const double* prm, int n) {
     return LDL_OK;
 }
 
-// Whether the layer transforms one mesh each way, the potential forward and the
-// divergence backward, with the derivatives taken in real space (k_grad6,
-// k_div6), or the three force and gradient spectra with the derivative symbol
-// applied in them.  One mesh is a third of the transform work (FP64 384^3
-// forward layer 9.05 -> 6.30 ms); FP32 meshes that are not powers of two keep
-// the symbol: differencing an FP32 potential rounds differently, which moves
-// their FP64-reduced gradients by up to 5e-8.
-template <typename T> inline bool layer_one_mesh(const Mesh& m) { return sizeof(T) == 8 || fft_mesh_pow2(m); }
-
 // Layer kinds: 0 sm, 1 dm, 2 HI (prm has 10 entries; star and S2buf used).
 enum { kKindSm = 0, kKindDm = 1, kKindHi = 2 };
 
@@ -1611,7 +1590,7 @@ static int sm_layer_fwd(int kind, const T* pos, const ldl_pos_desc* pdesc, int64
     // 3. x pass + filter + inverse x pass (and the x difference)
     const SmFilter<T> fl = layer_filter<T>(prm, kind == kKindDm);
     const T a1e2 = (T)((hi ? 1e-3 : 1e-2) * prm[0]);
-    if (x_pow2<T>(m)) {
+    if (fft_mesh_pow2(m)) {
         dispatch_n(m.n0, [&](auto N) {
             constexpr int NN = decltype(N)::value;
             ColGeom g = col_geom<T, NN>(m.n1, nh, hp, m.n1 * hp);
@@ -1636,7 +1615,7 @@ static int sm_layer_fwd(int kind, const T* pos, const ldl_pos_desc* pdesc, int64
             else run(&k_sm_x_any_fwd<T, XP, false>);
         });
         if (rc) return rc;
-    } else if constexpr (sizeof(T) == 4) {
+    } else {
         if ((rc = colpass<T, -1>(m.n0, m.n1, nh, hp, m.n1 * hp, tw, PlainColOp<T>{U, U, invM}, st))) return rc;
         const unsigned gf = grid_for(hc, 256, 1 << 16);
         if (hi)
@@ -1647,7 +1626,7 @@ static int sm_layer_fwd(int kind, const T* pos, const ldl_pos_desc* pdesc, int64
             if ((rc = colpass<T, +1>(m.n0, m.n1, nh, hp, m.n1 * hp, tw, PlainColOp<T>{P.spec3 + d * hc, P.spec3 + d * hc, T(1)}, st))) return rc;
     }
     // 4. inverse y passes (3 force spectra as 3*N0 planes) and z c2r into F
-    if (layer_one_mesh<T>(m)) {  // phi = inverse transform of P (x pass output in slot 0), F = -grad6(phi)
+    if (fft_mesh_pow2(m)) {  // phi = inverse transform of P (x pass output in slot 0), F = -grad6(phi)
         T* phi = P.mesh3;
         if ((rc = colpass<T, +1>(m.n1, m.n0, nh, m.n1 * hp, hp, tw, PlainColOp<T>{P.spec3, P.spec3, T(1)}, st))) return rc;
         if ((rc = zpass_c2r<T>(nrows, m.n2, tw, HalfRowLoad<T>{P.spec3, hp}, RealRowStore<T>{phi, m.n2, T(1)}, st, nullptr)))
@@ -1711,7 +1690,7 @@ static int sm_layer_bwd(int kind, const T* pos, const ldl_pos_desc* pdesc, int64
     // 2. unnormalised r2c of the real-space divergence of the three meshes
     // (layer_one_mesh: one spectrum, slot 0), else of the three meshes (z and y
     // passes; the filter kernel applies the i D_d)
-    if (layer_one_mesh<T>(m)) {
+    if (fft_mesh_pow2(m)) {
         T* dv = reinterpret_cast<T*>(P.spec3 + 2 * hc);  // a real mesh in the free third spectrum
         launch_div6<T>(m, P.mesh3, dv, (T)((double)m.n0 / (60.0 * pdesc->box[0])), (T)((double)m.n1 / (60.0 * pdesc->box[1])),
                        (T)((double)m.n2 / (60.0 * pdesc->box[2])), st);
@@ -1741,7 +1720,7 @@ static int sm_layer_bwd(int kind, const T* pos, const ldl_pos_desc* pdesc, int64
     const int64_t zdbl = std::min<int64_t>(m.n1 / 2, nh);  // end of c2f's doubled z bins (reference rule)
     c2<T>* S = P.spec3;  // result reuses the first spectrum (read before written)
     int64_t ntx = 0;
-    if (x_pow2<T>(m)) {
+    if (fft_mesh_pow2(m)) {
         dispatch_n(m.n0, [&](auto N) {
             constexpr int NN = decltype(N)::value;
             ColGeom g = col_geom<T, NN, xbwd_pencils<T, NN>()>(m.n1, nh, hp, m.n1 * hp);
@@ -1769,7 +1748,7 @@ static int sm_layer_bwd(int kind, const T* pos, const ldl_pos_desc* pdesc, int64
             else run(&k_sm_x_any_bwd<T, XP, false>);
         });
         if (rc) return rc;
-    } else if constexpr (sizeof(T) == 4) {
+    } else {
         for (int d = 0; d < 3; d++)
             if ((rc = colpass<T, -1>(m.n0, m.n1, nh, hp, m.n1 * hp, tw, PlainColOp<T>{P.spec3 + d * hc, P.spec3 + d * hc, T(1)}, st))) return rc;
         const unsigned gf = grid_for(hc, 256, 4096);
