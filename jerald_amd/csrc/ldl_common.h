@@ -8,6 +8,7 @@
 #include <string>
 
 #include "../../include/ldl.h"
+#include "posmath.h"
 #include "pow64.h"
 
 namespace ldl {
@@ -60,34 +61,6 @@ __host__ __device__ __forceinline__ int64_t wrapi(int64_t i, int64_t n) {
     if (i == -1) return n - 1;
     int64_t r = i % n;
     return r < 0 ? r + n : r;
-}
-
-// a / b, correctly rounded as the IEEE division, for positive normal b and y =
-// RN(1 / b): two corrections of a y with exact residuals (Markstein, IBM J.
-// Res. Dev. 34, 1990: one from a faithful quotient rounds correctly; the first
-// makes it faithful).  Five operations instead of the division's dozen.  Tiny
-// a, whose residuals could underflow, and y = 0 divide.
-template <typename T> __device__ __forceinline__ T div_by_cell(T a, T b, T y) {
-    constexpr T tiny = sizeof(T) == 4 ? T(1e-25) : T(1e-250);
-    if (!(a >= tiny) || y == T(0)) return a / b;
-    T q = a * y;
-    q = fma(fma(-b, q, a), y, q);
-    return fma(fma(-b, q, a), y, q);
-}
-
-// fmod(|r|, b) with the sign of r, b > 0: exact as fmod is (each difference of
-// two numbers within a factor of two is), in a few instructions a binary digit
-// of |r| / b; NaN for an infinite r.  The library's loop costs a kernel some 20
-// registers.
-template <typename T> __device__ __forceinline__ T fmod_digits(T r, T b) {
-    T a = fabs(r);
-    if (!(a < T(INFINITY))) return T(NAN);
-    while (a >= b) {
-        T s = ldexp(b, ilogb(a) - ilogb(b));
-        if (s > a) s *= T(0.5);
-        a -= s;
-    }
-    return copysign(a, r);
 }
 
 // ------------------------------------------------------ position decoding
