@@ -65,6 +65,8 @@ typedef struct ldl_pos_desc {
                                     earlier forward of them); the density paint reads it instead of
                                     sorting (same bits).  No counterpart in the reference: a backward
                                     pass that recomputes a layer keeps the forward's sort. */
+#define LDL_PAINT_LATTICE 16     /* workspace queries: the positions are LDL_POS_LATTICE, whose sort
+                                    keeps no lists of particles out of order (the paints ignore it) */
 
 const char* ldl_last_error(void);
 int ldl_version(void);
@@ -93,11 +95,13 @@ int ldl_buildplan(const int64_t nmesh[3], int32_t out[2]);
 /* ----------------------------------------------------------------- paint */
 /* Workspace for a paint of ``ncomp`` (1 or 3) components of ``np`` particles
  * with paint ``flags``: the particle sort's keys and indices (8 B per particle
- * plus 64 B per 8x16x32-cell tile) and, from 2^22 particles on, its lists of
- * particles out of order (12 B per particle and up to 8 MB; a smaller workspace
- * without room for them is accepted: the sort then does without);
- * LDL_PAINT_DIRECT adds the 64-bit accumulator mesh (8 B per cell and
- * component); LDL_PAINT_FLOAT_ATOMIC needs none (0). */
+ * plus 64 B per 8x16x32-cell tile) and, from 2^22 absolute positions on, its
+ * lists of particles out of order (12 B per particle and up to 8 MB).  Lattice
+ * positions need no lists: with LDL_PAINT_LATTICE the size is without.  A
+ * workspace of that size is accepted for absolute positions too, whose sort
+ * then does without lists (slower where many particles are out of order, same
+ * bits).  LDL_PAINT_DIRECT adds the 64-bit accumulator mesh (8 B per cell and
+ * component) and has no lists; LDL_PAINT_FLOAT_ATOMIC needs none (0). */
 size_t ldl_paint_workspace_bytes(const int64_t nmesh[3], int32_t ncomp, int64_t np, int32_t flags);
 
 /* Replaces ppaint_f32/_f64 (lib/cpu.cc:51-72 -> lib/parops_fast.h:483-531).
@@ -115,8 +119,8 @@ int ldl_ppaint_f64(const double* pos, const ldl_pos_desc* pd, int64_t np, const 
  * serving loops, harnesses that forbid hipMalloc).  Same arguments, output
  * and bits as ldl_ppaint_*; the workspace is a fixed 64 MiB array in the
  * library's device memory (one per GPU, held until the process ends), which
- * covers ldl_paint_workspace_bytes(nmesh, 1, np, flags) up to 64 MiB (with
- * the tiled paint: 8.1e6 particles on a 512^3 mesh, 6.3e6 on 1024^3);
+ * covers ldl_paint_workspace_bytes(nmesh, 1, np, flags | LDL_PAINT_LATTICE) up
+ * to 64 MiB (with the tiled paint: 8.1e6 particles on a 512^3 mesh, 6.3e6 on 1024^3);
  * larger requests return LDL_EINVAL.  Calls that overlap on one GPU (concurrent streams or
  * threads) share that array and race: serialise them.  LDL_PAINT_WS_ZEROED is
  * ignored (the array keeps the previous call's contents, so it is cleared).
@@ -205,7 +209,12 @@ int ldl_spectrum_zweight_f64(const double* in, double* out, const int64_t nmesh[
  * (model.py:268-272):  rho = fact * paint(X, 1); U = r2c((rho+1e-8)^gamma);
  * P = 1e-2 alpha G(k) U with G = -exp(-k^2/kl^2 - kh^2/k^2) k^nu;
  * F_d = c2r(-i D_d(k) P) with D_d the 6th-order FD symbol; s_d = readout(X, F_d).
- * Positions are LDL_POS_LATTICE displacements (mesh units) or physical. */
+ * Positions are LDL_POS_LATTICE displacements (mesh units) or physical.
+ * The workspace: the 3-component paint's without lists, three half spectra,
+ * three meshes, axis tables and partial sums.  The lists of a sort of absolute
+ * positions lie in the spectra's room, which the query widens to hold them;
+ * with LDL_PAINT_LATTICE in paint_flags it does not, and a workspace of that
+ * size is accepted for absolute positions too (lists if they fit). */
 size_t ldl_sm_workspace_bytes(const int64_t nmesh[3], int32_t is_f64, int64_t np, int32_t paint_flags);
 
 /* Size of a layer's particle sort (tile offsets + sorted indices + the FP32

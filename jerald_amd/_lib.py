@@ -21,6 +21,7 @@ LDL_PAINT_FLOAT_ATOMIC = 1
 LDL_PAINT_WS_ZEROED = 2
 LDL_PAINT_DIRECT = 4
 LDL_PAINT_BINS_VALID = 8
+LDL_PAINT_LATTICE = 16
 
 
 class LdlError(RuntimeError):

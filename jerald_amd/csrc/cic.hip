@@ -108,12 +108,12 @@ struct PaintWs {
     bool strays;
 };
 static bool paint_direct(int32_t flags) { return (flags & LDL_PAINT_DIRECT) && !(flags & LDL_PAINT_FLOAT_ATOMIC); }
-static PaintWs paint_ws(const Mesh& m, int nc, int64_t np, int32_t flags, const TileGeom& tg, bool lists = true) {
+static PaintWs paint_ws(const Mesh& m, int nc, int64_t np, int32_t flags, const TileGeom& tg, bool lists) {
     const int64_t nk = tg.nkeys();
     PaintWs w;
     w.acc = al256((size_t)kHdrBytes);
     w.counts = w.acc + (paint_direct(flags) ? al256((size_t)nc * m.cells() * 8) : 0);
-    w.strays = lists && np >= kStrayMin && nk <= ((int64_t)kBins << kBinKeysLog);
+    w.strays = lists && !paint_direct(flags) && np >= kStrayMin && nk <= ((int64_t)kBins << kBinKeysLog);
     w.bins = w.counts + (size_t)nk * 4;  // cleared together
     w.offsets = w.counts + al256((size_t)(nk + 1 + (w.strays ? kBins : 0)) * 4);
     w.segsum = w.offsets + al256((size_t)(nk + 1) * 4);
@@ -130,7 +130,7 @@ static PaintWs paint_ws(const Mesh& m, int nc, int64_t np, int32_t flags, const 
 size_t paint_ws_bytes(const Mesh& m, int nc, int64_t np, int32_t flags) {
     if (flags & LDL_PAINT_FLOAT_ATOMIC) return 0;  // float atomics deposit straight into the output
     np = np < 0 ? 0 : np;
-    return paint_ws(m, nc, np, flags, paint_tiles(m, np, nc == 3).tg).total;
+    return paint_ws(m, nc, np, flags, paint_tiles(m, np, nc == 3).tg, !(flags & LDL_PAINT_LATTICE)).total;
 }
 
 size_t paint_bins_bytes(const Mesh& m, int64_t np) {
@@ -176,10 +176,11 @@ int paint_impl(const T* pos, const ldl_pos_desc* pdesc, int64_t np, const T* mas
     }
     if (np > (int64_t)0xFFFFFFFFll) return fail(LDL_EUNSUPPORTED, "paint supports np < 2^32");
     // a workspace without room for the stray lists (ldl_ppaint_noalloc's fixed
-    // one) or the flat tiles' keys sorts without them
+    // one, or one sized for lattice positions) or the flat tiles' keys sorts
+    // without them
     const bool wide = sizeof(T) == 8 ? nc == 3 || bins_in || bins_out : nc == 3 && !wmesh;
     PaintTiles pt = paint_tiles(m, np, wide);
-    PaintWs w = paint_ws(m, nc, np, flags, pt.tg);
+    PaintWs w = paint_ws(m, nc, np, flags, pt.tg, pd.physical());
     if (ws && ws_bytes < w.total) w = paint_ws(m, nc, np, flags, pt.tg, false);
     if (ws && ws_bytes < w.total && !bins_in && !bins_out) {
         pt = paint_tiles(m, np, wide, false);
@@ -261,11 +262,10 @@ int paint_impl(const T* pos, const ldl_pos_desc* pdesc, int64_t np, const T* mas
         sorted = bins_out + nk + 1;
         if (nc == 1 && sizeof(T) == 4) vmax_out = bins_out + nk + 1 + np;
     }
-    const bool strays = w.strays && pd.physical();
     pp.vmax_out = vmax_out;
     if (!bins_in) {
         pp.counts = counts;
-        pp.ncounts = nk + (strays ? kBins : 0);
+        pp.ncounts = nk + (w.strays ? kBins : 0);
     } else if (nc == 3 && sizeof(T) == 4 && wmesh) {
         // recorded by the 1-component paint that wrote the sort and wmesh
         pp.vmax_in = bins_in + nk + 1 + np;
@@ -280,18 +280,18 @@ int paint_impl(const T* pos, const ldl_pos_desc* pdesc, int64_t np, const T* mas
         const bool few = np < kFew;
         const int64_t nchunks = few ? (np + 256 * kFewPPT - 1) / (256 * kFewPPT) : sort_chunks(np);
         StrayLists sl{};
-        if (strays) {
+        if (w.strays) {
             auto u = [&](size_t off) { return reinterpret_cast<unsigned*>(wb + off); };
             sl = StrayLists{u(w.list), reinterpret_cast<uint2*>(wb + w.pair), u(w.seg), u(w.off), u(w.bins), stray_group_size(np), 0};
             while (((int64_t)kBins << sl.shift) < nk) sl.shift++;
         }
-        const dim3 gb(strays ? (unsigned)stray_groups(np) : grid_for(nchunks, 1, 1 << 15));
+        const dim3 gb(w.strays ? (unsigned)stray_groups(np) : grid_for(nchunks, 1, 1 << 15));
         if (np > 0) {
             KTimer _t("paint_bin", st);
             with_dm([&](auto D) {
                 constexpr int DM = decltype(D)::value;
                 if constexpr (DM == kDecPhysP2 || DM == kDecPhys) {
-                    if (strays) {
+                    if (w.strays) {
                         hipLaunchKernelGGL((k_bin_keys<T, kSortPPT, DM, true>), gb, dim3(256), 0, st, pos, pd, np, mp, tg, counts, key, sl);
                         return;
                     }
@@ -299,7 +299,7 @@ int paint_impl(const T* pos, const ldl_pos_desc* pdesc, int64_t np, const T* mas
                 if (few) hipLaunchKernelGGL((k_bin_keys<T, kFewPPT, DM, false>), gb, dim3(256), 0, st, pos, pd, np, mp, tg, counts, key, sl);
                 else hipLaunchKernelGGL((k_bin_keys<T, kSortPPT, DM, false>), gb, dim3(256), 0, st, pos, pd, np, mp, tg, counts, key, sl);
             });
-            if (strays) {
+            if (w.strays) {
                 hipLaunchKernelGGL(k_stray_part, gb, dim3(kStrayThreads), 0, st, key, sl);
                 hipLaunchKernelGGL(k_stray_count, dim3(1024), dim3(kStrayThreads), 0, st, sl, counts);
             }
@@ -314,8 +314,8 @@ int paint_impl(const T* pos, const ldl_pos_desc* pdesc, int64_t np, const T* mas
             KTimer _t("paint_scatter", st);
             const dim3 gs(grid_for(nchunks, 1, 1 << 15));
             if (few) hipLaunchKernelGGL(k_bin_scatter<kFewPPT>, gs, dim3(256), 0, st, np, key, 0u, counts, sorted);
-            else hipLaunchKernelGGL(k_bin_scatter<kSortPPT>, gs, dim3(256), 0, st, np, key, strays ? kStrayBit : 0u, counts, sorted);
-            if (strays) hipLaunchKernelGGL(k_stray_scatter, dim3(1024), dim3(kStrayThreads), 0, st, sl, counts, sorted);
+            else hipLaunchKernelGGL(k_bin_scatter<kSortPPT>, gs, dim3(256), 0, st, np, key, w.strays ? kStrayBit : 0u, counts, sorted);
+            if (w.strays) hipLaunchKernelGGL(k_stray_scatter, dim3(1024), dim3(kStrayThreads), 0, st, sl, counts, sorted);
         }
     }
     if (nc == 3 && sizeof(T) == 4 && wmesh && !bins_in) {

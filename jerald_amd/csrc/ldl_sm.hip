@@ -134,9 +134,11 @@ struct SmWs {
 static SmWs sm_ws(const Mesh& m, int tsize, int64_t np, int32_t pflags) {
     auto al = [](size_t b) { return (b + 255) & ~(size_t)255; };
     SmWs w;
-    w.paint = al(paint_ws_bytes(m, 3, np, pflags));
+    w.paint = al(paint_ws_bytes(m, 3, np, pflags | LDL_PAINT_LATTICE));
     const int64_t hq = (64 / (2 * tsize)), hcp = m.n0 * m.n1 * ((m.nh() + hq - 1) / hq * hq);  // spec_cells
-    w.spec3 = al((size_t)3 * hcp * 2 * tsize);
+    // also holds the stray lists of the sort, which follow the paint region:
+    // both paints are done before a spectrum is written
+    w.spec3 = std::max(al((size_t)3 * hcp * 2 * tsize), al(paint_ws_bytes(m, 3, np, pflags)) - w.paint);
     // three meshes; also holds one pitched spectrum (the HI layer's T2)
     w.mesh3 = al((size_t)std::max<int64_t>(3 * m.cells(), 2 * hcp) * tsize);
     w.tabs = al((size_t)2 * (m.n0 + m.n1 + m.nh()) * tsize);
@@ -144,6 +146,17 @@ static SmWs sm_ws(const Mesh& m, int tsize, int64_t np, int32_t pflags) {
     w.part = al((size_t)w.part_doubles * 8);
     w.total = w.paint + w.spec3 + w.mesh3 + w.tabs + w.part;
     return w;
+}
+
+// The same of a layer's workspace: lattice positions need no room for lists, and
+// absolute ones do without where there is none.
+template <typename T>
+static int layer_ws(const Mesh& m, const PosDec<T>& pd, int64_t np, int32_t pflags, const void* ws, size_t wsb, SmWs* w) {
+    if (!pd.physical()) pflags |= LDL_PAINT_LATTICE;
+    *w = sm_ws(m, sizeof(T), np, pflags);
+    if (wsb < w->total) *w = sm_ws(m, sizeof(T), np, pflags | LDL_PAINT_LATTICE);
+    if (!ws || wsb < w->total) return fail(LDL_EINVAL, "sm workspace too small (see ldl_sm_workspace_bytes)");
+    return LDL_OK;
 }
 
 template <typename T> struct SmPtrs {
@@ -1558,8 +1571,8 @@ static int sm_layer_fwd(int kind, const T* pos, const ldl_pos_desc* pdesc, int64
     PosDec<T> pd;
     if ((rc = make_posdec<T>(pdesc, nmesh, np, &pd))) return rc;
     const Sweep sw = make_sweep(pd, np);
-    const SmWs w = sm_ws(m, sizeof(T), np, pflags);
-    if (!ws || wsb < w.total) return fail(LDL_EINVAL, "sm workspace too small (see ldl_sm_workspace_bytes)");
+    SmWs w;
+    if ((rc = layer_ws(m, pd, np, pflags, ws, wsb, &w))) return rc;
     const SmPtrs<T> P = sm_ptrs<T>(ws, w);
     const c2<T>* tw;
     if ((rc = twiddles<T>(&tw))) return rc;
@@ -1569,7 +1582,7 @@ static int sm_layer_fwd(int kind, const T* pos, const ldl_pos_desc* pdesc, int64
     const bool bins_in = tiled && bins && (pflags & LDL_PAINT_BINS_VALID);
     AxisTabs<T> at;  // filled by the paint's first launch
     const KTabs<T> kt = axis_tables<T>(P.tabs, m, pdesc->box, &at);
-    if ((rc = paint_impl<T>(pos, pdesc, np, nullptr, 1.0, 1, nmesh, fact, pflags & ~LDL_PAINT_BINS_VALID, rho, P.paint, w.paint, st,
+    if ((rc = paint_impl<T>(pos, pdesc, np, nullptr, 1.0, 1, nmesh, fact, pflags & ~LDL_PAINT_BINS_VALID, rho, P.paint, w.paint + w.spec3, st,
                             tiled && !bins_in ? reinterpret_cast<unsigned*>(bins) : nullptr,
                             bins_in ? reinterpret_cast<const unsigned*>(bins) : nullptr, nullptr, 0.0, nullptr, false, at)))
         return rc;
@@ -1671,8 +1684,8 @@ static int sm_layer_bwd(int kind, const T* pos, const ldl_pos_desc* pdesc, int64
     PosDec<T> pd;
     if ((rc = make_posdec<T>(pdesc, nmesh, np, &pd))) return rc;
     const Sweep sw = make_sweep(pd, np);
-    const SmWs w = sm_ws(m, sizeof(T), np, pflags);
-    if (!ws || wsb < w.total) return fail(LDL_EINVAL, "sm workspace too small (see ldl_sm_workspace_bytes)");
+    SmWs w;
+    if ((rc = layer_ws(m, pd, np, pflags, ws, wsb, &w))) return rc;
     const SmPtrs<T> P = sm_ptrs<T>(ws, w);
     const c2<T>* tw;
     if ((rc = twiddles<T>(&tw))) return rc;
@@ -1684,7 +1697,7 @@ static int sm_layer_bwd(int kind, const T* pos, const ldl_pos_desc* pdesc, int64
     // for the maxima of g_in
     AxisTabs<T> at;
     const KTabs<T> kt = axis_tables<T>(P.tabs, m, pdesc->box, &at);
-    if ((rc = paint_impl<T>(pos, pdesc, np, gout, 0.0, 3, nmesh, 1.0, pflags, P.mesh3, P.paint, w.paint, st, nullptr,
+    if ((rc = paint_impl<T>(pos, pdesc, np, gout, 0.0, 3, nmesh, 1.0, pflags, P.mesh3, P.paint, w.paint + w.spec3, st, nullptr,
                             reuse ? reinterpret_cast<const unsigned*>(bins) : nullptr, rho, 1.0 / fact, gmax, np > 0, at)))
         return rc;
     // 2. unnormalised r2c of the real-space divergence of the three meshes

@@ -145,9 +145,12 @@ class JERALDModel:
         return L.pos_desc(self.box, L.LDL_POS_LATTICE, self.lattice, step)
 
     # ------------------------------------------------------- kernels
+    def _ws_flags(self):
+        return self.paint_flags | (L.LDL_PAINT_LATTICE if self.lattice is not None else 0)
+
     def _ws(self):
         np_ = 0 if self.X is None else self.X.shape[0]
-        nb = L.load().ldl_sm_workspace_bytes(L.i64x3(self.nm), int(self.dtype == torch.float64), np_, self.paint_flags)
+        nb = L.load().ldl_sm_workspace_bytes(L.i64x3(self.nm), int(self.dtype == torch.float64), np_, self._ws_flags())
         return L.workspaces.get(self.device, f"sm{self.dtype}", nb)
 
     def _layer_fwd(self, P, prm, fact, keep_bins=False, need_out=True, bins=None):
@@ -183,7 +186,7 @@ class JERALDModel:
     def _paint_density(self, P, fact):
         dt, dev, nm = self.dtype, self.device, self.nm
         rho = torch.empty(nm, dtype=dt, device=dev)
-        nb = L.load().ldl_paint_workspace_bytes(L.i64x3(nm), 1, P.shape[0], self.paint_flags)
+        nb = L.load().ldl_paint_workspace_bytes(L.i64x3(nm), 1, P.shape[0], self._ws_flags())
         ws = L.workspaces.get(dev, f"paint1", nb)
         L.call(f"ldl_ppaint_{L.sfx(dt)}", L.ptr(P), self._pd(), P.shape[0], None, 1.0, L.i64x3(nm), float(fact),
                self.paint_flags, L.ptr(rho), L.ptr(ws), ws.numel(), L.stream_ptr(dev))
