@@ -95,7 +95,8 @@ int ldl_buildplan(const int64_t nmesh[3], int32_t out[2]);
 /* ----------------------------------------------------------------- paint */
 /* Workspace for a paint of ``ncomp`` (1 or 3) components of ``np`` particles
  * with paint ``flags``: the particle sort's keys and indices (8 B per particle
- * plus 64 B per 8x16x32-cell tile) and, from 2^22 absolute positions on, its
+ * plus 64 B per 8x16x32-cell tile; eight or two times that many smaller tiles
+ * where these are faster, for which a workspace may lack the room) and, from 2^22 absolute positions on, its
  * lists of particles out of order (12 B per particle and up to 8 MB).  Lattice
  * positions need no lists: with LDL_PAINT_LATTICE the size is without.  A
  * workspace of that size is accepted for absolute positions too, whose sort

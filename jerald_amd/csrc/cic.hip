@@ -81,8 +81,10 @@ static inline int64_t stray_group_size(int64_t np) { return (sort_chunks(np) + s
 // FP32 339 -> 281; FP64 one component (256 threads) 223 -> 205.  The 32-bit
 // paints have that occupancy with the longer z runs, and the FP64 one-component
 // paint on its own keeps the workspace it had.  Meshes whose keys would
-// no longer fit the stray lists (FP64 at 1024^3) keep the large tiles, and so
-// does a workspace with no room for twice the keys.
+// no longer fit the stray lists (FP64 at 1024^3) keep the large tiles.
+//
+// A workspace with room for the large tiles' keys alone takes those in place of
+// either split.
 template <int N> using Int = std::integral_constant<int, N>;
 enum Split { kSplitLarge, kSplitSmall, kSplitFlat };
 static constexpr int kSmallX = 4, kSmallY = 8, kSmallZ = 16, kSmallBlock = 256;
@@ -91,11 +93,12 @@ struct PaintTiles {
     TileGeom tg;
     Split split;
 };
-static PaintTiles paint_tiles(const Mesh& m, int64_t np, bool wide, bool flat = true) {
+static PaintTiles paint_tiles(const Mesh& m, int64_t np, bool wide, bool large_only = false) {
     static const int large[3] = {3, 4, 5}, small[3] = {2, 3, 4}, flats[3] = {3, 4, 4};
     const TileGeom tg = make_tiles(m, large);
+    if (large_only) return {tg, kSplitLarge};
     if (tg.ntiles < 256 && np < kStrayMin) return {make_tiles(m, small), kSplitSmall};
-    if (!wide || !flat) return {tg, kSplitLarge};
+    if (!wide) return {tg, kSplitLarge};
     const TileGeom tf = make_tiles(m, flats);
     if (tf.nkeys() > ((int64_t)kBins << kBinKeysLog)) return {tg, kSplitLarge};
     return {tf, kSplitFlat};
@@ -176,14 +179,14 @@ int paint_impl(const T* pos, const ldl_pos_desc* pdesc, int64_t np, const T* mas
     }
     if (np > (int64_t)0xFFFFFFFFll) return fail(LDL_EUNSUPPORTED, "paint supports np < 2^32");
     // a workspace without room for the stray lists (ldl_ppaint_noalloc's fixed
-    // one, or one sized for lattice positions) or the flat tiles' keys sorts
+    // one, or one sized for lattice positions) or the smaller tiles' keys sorts
     // without them
     const bool wide = sizeof(T) == 8 ? nc == 3 || bins_in || bins_out : nc == 3 && !wmesh;
     PaintTiles pt = paint_tiles(m, np, wide);
     PaintWs w = paint_ws(m, nc, np, flags, pt.tg, pd.physical());
     if (ws && ws_bytes < w.total) w = paint_ws(m, nc, np, flags, pt.tg, false);
     if (ws && ws_bytes < w.total && !bins_in && !bins_out) {
-        pt = paint_tiles(m, np, wide, false);
+        pt = paint_tiles(m, np, wide, true);
         w = paint_ws(m, nc, np, flags, pt.tg, false);
     }
     if (!ws || ws_bytes < w.total) return fail(LDL_EINVAL, "paint workspace too small (see ldl_paint_workspace_bytes)");
