@@ -96,18 +96,7 @@ template <typename T> struct PosDec {
         base[0] = base[1] = base[2] = 0;
         if (PHYS || kind == LDL_POS_PHYSICAL) {
 #pragma unroll
-            for (int d = 0; d < 3; d++) {
-                // numpy remainder semantics, then division (jaxpops_bind.py:163-164);
-                // fmod is the identity on [0, L), exactly r - L on [L, 2L)
-                // and the identity again on (-L, 0), where L is added
-                T r = x[d];
-                if (!(r >= T(0) && r < box[d])) {
-                    if (r >= box[d] && r < T(2) * box[d]) r -= box[d];
-                    else if (!(r > -box[d] && r < T(0))) r = fmod_digits(r, box[d]);
-                    if (r < T(0)) r += box[d];
-                }
-                x[d] = div_by_cell(r, cell[d], cellrcp[d]);
-            }
+            for (int d = 0; d < 3; d++) x[d] = mesh_coordinate(x[d], box[d], cell[d], cellrcp[d]);
         } else {
             uint32_t pp = (uint32_t)p;
             uint32_t li[3];
@@ -221,11 +210,11 @@ inline int make_posdec(const ldl_pos_desc* pd, const int64_t nmesh[3], int64_t n
     out->kind = pd->kind;
     for (int d = 0; d < 3; d++) {
         if (!(pd->box[d] > 0.0) || !std::isfinite(pd->box[d])) return fail(LDL_EINVAL, "box sizes must be positive and finite");
-        out->box[d] = (T)pd->box[d];
+        out->box[d] = period_of<T>(pd->box[d]);
         out->cell[d] = out->box[d] / (T)nmesh[d];
         constexpr double span = sizeof(T) == 4 ? 1e12 : 1e100;
         out->cellrcp[d] = (double)out->cell[d] > 1 / span && (double)out->cell[d] < span ? T(1) / out->cell[d] : T(0);
-        out->cellinv[d] = (T)nmesh[d] / out->box[d];
+        out->cellinv[d] = (T)nmesh[d] / (T)pd->box[d];
         out->n[d] = nmesh[d];
         out->lstep[d] = pd->lattice_step[d];
     }

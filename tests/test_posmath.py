@@ -1,6 +1,6 @@
 """The position decode's remainder and division against the C library's fmod
 and the IEEE division, compiled for the CPU: ordinary and extreme ratios,
-subnormal and infinite arguments, and a period that rounded to zero."""
+subnormal and infinite arguments, and boxes that round to zero."""
 import os
 import subprocess
 
@@ -26,7 +26,15 @@ template <typename T> int check(const char* name) {
     const T edge[] = {T(0), -T(0), T(1), L::min(), L::denorm_min(), L::max(), L::infinity(), L::quiet_NaN(), T(51.3), T(-409.6)};
     for (T r : edge)
         for (T b : edge)
-            if (!(b < T(0)) && b < L::infinity() && !std::signbit(b)) rem(r, b);
+            if (b > T(0) && b < L::infinity()) rem(r, b);
+    for (double box : {51.3, 1e-46, 4e-324, 1e-40, 409.6})  // some round to zero in T
+        for (T r : edge) {
+            const T L = ldl::period_of<T>(box), cell = L / 20;
+            T u = std::fmod(r, (T)box);
+            if (u < T(0)) u += (T)box;
+            const T got = ldl::mesh_coordinate(r, L, cell, cell > T(1e-12) ? T(1) / cell : T(0));
+            if (!same(got, u / ((T)box / 20)) && bad++ < 5) std::printf("%s coordinate %a in %g\n", name, (double)r, box);
+        }
     for (int i = 0; i < 200000; i++) {
         const T b = std::ldexp((T)(1.5 + 0.5 * u(g)), (int)(20 * u(g)));
         rem((T)(u(g) * std::pow(2.0, 60 * u(g))) * b, b);
