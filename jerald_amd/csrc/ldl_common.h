@@ -157,10 +157,11 @@ template <typename T> struct PosDec {
             }
         }
     }
-    // base + fl wrapped into [0, n), base < n: in 32 bits up to one period off
-    // (a negative sum wraps to 2^31 or more, above every n), else as wrapi.
+    // base + fl wrapped into [0, n): in 32 bits for base below 2^31 up to one
+    // period off (a negative sum wraps to 2^31 or more, above every n), else as
+    // wrapi.
     static __device__ __forceinline__ uint32_t wrap_cell(T fl, uint32_t base, int64_t n) {
-        if (fabs(fl) < T(1 << 29)) {
+        if (fabs(fl) < T(1 << 29) && base < (1u << 31)) {
             const uint32_t u = base + (uint32_t)(int32_t)fl, m = (uint32_t)n;
             if (u < m) return u;
             const uint32_t v = fl < T(0) ? u + m : u - m;
@@ -233,6 +234,9 @@ inline int make_posdec(const ldl_pos_desc* pd, const int64_t nmesh[3], int64_t n
         out->sh2 = lg(out->l2);
         for (int d = 0; d < 3; d++)
             if (!(pd->lattice_step[d] > 0.0)) return fail(LDL_EINVAL, "lattice_step must be positive");
+        // cell numbers are 32-bit: whole periods come out of steps that lead beyond
+        for (int d = 0; d < 3; d++)
+            if (pd->lattice_step[d] * (double)(pd->lattice[d] - 1) >= (double)(1u << 31)) out->lstep[d] = std::fmod(pd->lattice_step[d], (double)nmesh[d]);
         out->unit = pd->lattice_step[0] == 1.0 && pd->lattice_step[1] == 1.0 && pd->lattice_step[2] == 1.0;
     }
     return LDL_OK;
