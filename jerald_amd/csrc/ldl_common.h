@@ -149,9 +149,9 @@ template <typename T> struct PosDec {
         for (int d = 0; d < 3; d++) {
             const T fl = floor(x[d]);
             f[d] = x[d] - fl;
-            if constexpr (PHYS) {  // 0 <= fl <= n (or NaN, which converts to 0)
+            if constexpr (PHYS) {  // 0 <= fl <= n, below 2 n where the cell size is subnormal (or NaN, which converts to 0)
                 const uint32_t u = (uint32_t)(int32_t)fl;
-                idx[d] = u < (uint32_t)n[d] ? u : 0u;
+                idx[d] = u < (uint32_t)n[d] ? u : u - (uint32_t)n[d] < (uint32_t)n[d] ? u - (uint32_t)n[d] : 0u;
             } else {
                 idx[d] = wrap_cell(fl, base[d], n[d]);
             }

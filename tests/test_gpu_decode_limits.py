@@ -42,3 +42,22 @@ def test_lattice_points_far_from_the_first(step, dtype):
     want = np.zeros(nm)
     np.add.at(want, tuple(idx), 1.0)
     assert np.array_equal(rho.double().cpu().numpy(), want)
+
+
+def test_subnormal_cells_wrap_as_the_division_rounds():
+    # L / N rounds by up to a part in a few: coordinates run past N and wrap
+    nm, L = (5, 6, 1000), np.float32(1e-41)
+    box = (float(L),) * 3
+    rng = np.random.default_rng(4)
+    x = (rng.random((500, 3)) * float(L) * 0.999).astype(np.float32)
+    u = x / (L / np.array(nm, dtype=np.float32))
+    assert u.dtype == np.float32 and (u[:, 2] > 1001).any()
+    i = np.floor(u).astype(int)
+    field = rng.standard_normal(nm).astype(np.float32)
+    want = np.zeros(500)
+    for a in range(8):
+        b = np.array([a >> 2, a >> 1, a]) & 1
+        w = np.prod(np.where(b, u - i, 1 - (u - i)).astype(float), axis=1)
+        want += w * field[tuple(((i + b) % nm).T)]
+    out = J.preadout(torch.tensor(x, device="cuda"), torch.tensor(field, device="cuda"), nm, box).double().cpu().numpy()
+    assert np.abs(out - want).max() <= 8 * np.finfo(np.float32).eps * np.abs(field).max()
