@@ -3,12 +3,15 @@
 // The FP64 layer passes that raise the density to gamma are bound by vector
 // instructions, not by memory, with library calls (each pow forms its own
 // extended logarithm; the gamma adjoint took two of them and a log).  Here
-// ln x = h + l is formed once to about 2^-60 and each power is one
-// exponential of a (h + l), within 0.58 ulp where a |ln x| <= 700 (the library pow:
-// 1.3 ulp over the same arguments).  256^3: gamma adjoint 287 -> 144 us, density
-// spectrum 132 -> 115.  Arguments
-// beyond that (zero, negative, subnormal, infinite and NaN bases, powers near
-// overflow or underflow) take the library's pow.
+// ln x = h + l is formed once to about 2^-63 of itself and each power is one
+// exponential of a (h + l).  The logarithm's error enters times |a ln x|: a power
+// is within 0.56 + |a ln x| / 1024 ulp where |a ln x| <= 700 (largest measured:
+// 0.57 ulp to |a ln x| = 128, 0.66 at 256, 1.08 at 700; the library's pow over
+// the same arguments: 1.34 from 4 on, 1.18 at 1).  h alone is the rounded
+// logarithm (0.501 ulp; the library's 0.65).  256^3: gamma adjoint 287 -> 144
+// us, density spectrum 132 -> 115.  Arguments beyond that (zero, negative,
+// subnormal, infinite and NaN bases, powers near overflow or underflow) take the
+// library's pow.
 //
 //   x = 2^e m, m in [sqrt(1/2), sqrt(2)), s = (m - 1) / (m + 1):
 //   ln m = 2 artanh s = 2 s + s^3 (2/3 + 2/5 s^2 + ...), |s| <= 0.172, the
@@ -43,7 +46,7 @@ LDL_HD double rcp_near(double d) {
 #endif
 }
 
-static constexpr double kLn2Hi = 0x1.62e42fefa38p-1;        // 40 bits: n kLn2Hi is exact for |n| < 2^12
+static constexpr double kLn2Hi = 0x1.62e42fefa38p-1;        // 42 bits: n kLn2Hi is exact for |n| < 2^11
 static constexpr double kLn2Lo = 0x1.ef35793c7673p-45;      // ln 2 - kLn2Hi
 
 // ln x for positive normal x.
