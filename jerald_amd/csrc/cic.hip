@@ -42,10 +42,15 @@ static inline size_t al256(size_t b) { return (b + 255) & ~(size_t)255; }
 
 // Stray lists (cic.h) for absolute positions, whose order is the caller's, from
 // 2^22 particles on, and on meshes whose keys fit their bins (1024^3 has 2^21
-// keys).  When every particle is in order they cost three empty launches and 3%
-// of the sort (512^3: 0.795 against 0.768 ms), with 40% of the particles in
-// clumps they take it from 6.8 to 2.6 ms.  Displacements from a lattice are in
-// order by construction and sort without.
+// keys).  When every particle is in order they cost three nearly empty launches
+// and the bins' scan, 7 to 25 us at any size (512^3: sort 0.768 -> 0.795 ms), so
+// below the line that is a quarter of the paint and more; out of order they pay
+// from 2^20 on, by the more the more particles there are.  FP32 paint, us,
+// without -> with lists, in order, 40% in clumps, shuffled: 2^20 particles on
+// 128^3 48 -> 66, 115 -> 86, 161 -> 93; 2^22 on 160^3 83 -> 104, 274 -> 193, 386
+// -> 239; 2^22 on 320^3 127 -> 142, 352 -> 216, 498 -> 267; 2^24 on 256^3 283 ->
+// 290, 1328 -> 615, 2541 -> 844.  Displacements from a lattice are in order by
+// construction and sort without.
 static constexpr int64_t kStrayMin = 1 << 22;
 static constexpr int kSortPPT = 8;  // particles per thread of the sort's passes: chunks of 2048
 // Below 2^20 particles (512 chunks of 2048, two per CU) chunks of 512 spread
@@ -54,6 +59,7 @@ static constexpr int kSortPPT = 8;  // particles per thread of the sort's passes
 // 128^3 takes 15 and 12 either way, 160^3 the scatter 16.6 -> 18.6.
 static constexpr int kFewPPT = 2;
 static constexpr int64_t kFew = 1 << 20;
+static_assert(kFew <= kStrayMin, "the scatter of few particles places every key, listed ones too");
 static inline int64_t sort_chunks(int64_t np) { return (np + 256 * kSortPPT - 1) / (256 * kSortPPT); }
 // Workgroups of the key pass with lists: two chunks each or more.
 static inline int64_t stray_groups(int64_t np) { return std::max<int64_t>(1, std::min<int64_t>(kSegs, sort_chunks(np) / 2)); }
