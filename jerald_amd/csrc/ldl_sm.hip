@@ -720,11 +720,10 @@ __global__ void __launch_bounds__(256) k_sm_filter_bwd(const c2<T>* S3, const c2
 // force spectra, hc apart, with the bits that the separate passes above also
 // give.  They are bound by the memory they move: one read of the tile and one
 // write per spectrum, where separate transforms and filter passes read and
-// wrote each spectrum twice more (384^3 FP32 forward 720 -> 423 us; FP64
-// one dm layer, loss and gradient 21.5 -> 20.6 ms).  A
-// thread holds elements q + s nq, s < 16, of column p between transforms:
-// in FP64 64 VGPRs beside the transform's 64, so it gets 256 and at most 512
-// threads share a workgroup.
+// wrote each spectrum twice more (384^3 FP32 forward 720 -> 423 us; FP64 loss
+// and gradient of one dm layer 21.5 -> 20.6 ms).  A thread holds elements q + s
+// nq, s < 16, of column p between transforms: in FP64 64 VGPRs beside the
+// transform's 64, so it gets 256 and at most 512 threads share a workgroup.
 template <typename T> constexpr int x_any_most() { return sizeof(T) == 4 ? 1024 : 512; }
 
 template <typename T, int P, bool HI>
@@ -1414,9 +1413,8 @@ template <typename T, bool PLAIN = false> struct LossSq2Store {
     }
 };
 
-// out = {loss / npix, g_mu, g_w, g_b, loss_v / npix_v[, g_zs]}
-// The loss columns' totals, and out = {loss, dL/dmu, dL/dw, dL/db, validation
-// loss (HI: , dL/dzs)} from them.
+// The loss columns' totals, and out = {loss / npix, dL/dmu, dL/dw, dL/db,
+// validation loss / npix_v (HI: , dL/dzs)} from them.
 __global__ void __launch_bounds__(kRedThreads) k_loss_finish(const double* __restrict__ part, int64_t nblocks, const double* __restrict__ npix,
                                                              double* __restrict__ out, int nout) {
     __shared__ double red[kRedCols][kRedThreads / 64], sums[kRedCols];

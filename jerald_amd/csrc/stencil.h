@@ -1,6 +1,7 @@
 // Real-space derivative stencils of the LDL layer on gfx950.
 #pragma once
 
+#include <algorithm>
 #include <type_traits>
 
 #include "ldl_common.h"
@@ -224,7 +225,7 @@ struct StCell {
         x = r / (uint32_t)g.n1;
     }
 };
-// circular neighbours v + k, k = -3..3 without 0, of v < n (any n >= 1)
+// circular neighbours v + k, k = -3..3 without 0, of v < n (n >= 3: one wrap)
 __device__ __forceinline__ void st_ring(uint32_t v, uint32_t n, uint32_t (&w)[6]) {
 #pragma unroll
     for (int k = 0; k < 6; k++) {
@@ -295,7 +296,7 @@ constexpr int64_t kStDirect = 1 << 20;
 // Marching tile and chunk: 64 cells wide below 2^24 cells (more, smaller
 // workgroups), else the width that pads n2 least, the widest on a tie (FP32
 // 384^3 grad6: 200 us at 128, 248 at 256); then the longest chunk of 64, 32,
-// 16, 8 or 4 planes that still gives 256 workgroups and 128 threads per CU
+// 16, 8 or 4 planes that still gives 256 workgroups and 512 threads per CU
 // (256^3 FP64: 128 x 32 planes 110 and 114 us, 64 planes 179 and 170).
 template <typename T>
 inline StGeom st_plan(const Mesh& m, int* tz) {
@@ -321,7 +322,7 @@ inline StGeom st_plan(const Mesh& m, int* tz) {
 
 template <typename T, class Direct, class March>
 inline void st_launch(const Mesh& m, Direct&& direct, March&& march) {
-    if (m.cells() <= kStDirect) {
+    if (m.cells() <= kStDirect && std::min(m.n0, std::min(m.n1, m.n2)) >= 3) {
         direct(st_geom<T>(m, 64, 64), (unsigned)((m.cells() + 255) / 256));
         return;
     }
