@@ -15,6 +15,8 @@ from jerald_amd.pmesh import PMesh
 pytestmark = pytest.mark.gpu
 
 MESHES = [(5, 8, 6), (45, 20, 30), (100, 12, 18), (360, 24, 20), (500, 16, 12), (972, 6, 10), (1000, 5, 6), (12, 96, 180), (64, 30, 20), (128, 16, 48)]
+# columns enough for the shapes that fill the chip (more than 4096 in FP64, 8192 in FP32)
+MANY = [(20, 96, 180), (240, 96, 180), (360, 64, 270), (640, 48, 180), (810, 60, 150), (960, 64, 144), (1000, 48, 180)]
 PRM = {"sm": [0.2, 0.7, 0.9, 4.0, 0.3], "dm": [0.2, 0.7, 0.9, 4.0, 0.3], "HI": [0.2, 0.7, 0.9, 4.0, 0.3, 0.1, 0.8, 1.1, 3.0, 0.2]}
 
 
@@ -32,6 +34,16 @@ def layer(nm, kind, dtype, X, star, v):
 @pytest.mark.parametrize("kind", ["sm", "dm", "HI"])
 @pytest.mark.parametrize("nm", MESHES, ids=str)
 def test_forces_and_adjoint_match_fp64(nm, kind):
+    compare(nm, kind)
+
+
+@pytest.mark.parametrize("kind", ["sm", "HI"])
+@pytest.mark.parametrize("nm", MANY, ids=str)
+def test_many_columns(nm, kind):
+    compare(nm, kind)
+
+
+def compare(nm, kind):
     rng = np.random.default_rng(21)
     q = np.stack(np.meshgrid(*[np.arange(n) for n in nm], indexing="ij"), -1).reshape(-1, 3)
     X = torch.tensor(np.mod(q + 0.4 * rng.standard_normal(q.shape), nm)).float()
