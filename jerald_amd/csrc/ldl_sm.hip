@@ -659,10 +659,9 @@ k_x_realfilter(ColGeom g, const c2<T>* __restrict__ tw, c2<T>* __restrict__ io, 
 // Layers whose x axis is a power of two and another axis is not run plain
 // column passes around the next two kernels; the loss smoothing of meshes whose
 // axes are not all powers of two runs them around k_realfilter_mult.  All go
-// over the half spectrum
-// (index i -> (ix, iy, iz) with iz fastest, rows of pitch hp; the pad columns
-// iz >= nh are skipped), which do what the fused x kernels do between their
-// transforms.
+// over the half spectrum (index i -> (ix, iy, iz) with iz fastest, rows of pitch
+// hp; the pad columns iz >= nh are skipped) and do what the fused x kernels do
+// between their transforms.
 
 // The three force spectra out3[d] = -i D_d P, P = cpot alpha G U [+ a G2 S2].
 template <typename T, bool HI>
@@ -1698,9 +1697,10 @@ static int sm_layer_bwd(int kind, const T* pos, const ldl_pos_desc* pdesc, int64
     if ((rc = paint_impl<T>(pos, pdesc, np, gout, 0.0, 3, nmesh, 1.0, pflags, P.mesh3, P.paint, w.paint + w.spec3, st, nullptr,
                             reuse ? reinterpret_cast<const unsigned*>(bins) : nullptr, rho, 1.0 / fact, gmax, np > 0, at)))
         return rc;
-    // 2. unnormalised r2c of the real-space divergence of the three meshes
-    // (layer_one_mesh: one spectrum, slot 0), else of the three meshes (z and y
-    // passes; the filter kernel applies the i D_d)
+    // 2. unnormalised r2c of the real-space divergence of the three meshes (one
+    // spectrum, slot 0) on a power-of-two mesh, else of the three meshes (z and
+    // y passes; the x pass applies the i D_d, whose products round less than
+    // differences of a rounded mesh)
     if (fft_mesh_pow2(m)) {
         T* dv = reinterpret_cast<T*>(P.spec3 + 2 * hc);  // a real mesh in the free third spectrum
         launch_div6<T>(m, P.mesh3, dv, (T)((double)m.n0 / (60.0 * pdesc->box[0])), (T)((double)m.n1 / (60.0 * pdesc->box[1])),

@@ -16,8 +16,8 @@ namespace ldl {
 // along axis d (circular): a circular shift by s multiplies transform bin n
 // by exp(+-2 pi i n s / N), so the transform of diff_d(a) / (60 h_d) is
 // i D_d times the transform of a, and the inverse transform of -i D_d P is
-// -diff_d(phi) / (60 h_d) with phi the inverse transform of P.  The layer
-// therefore transforms one mesh each way: k_grad6 turns the potential phi
+// -diff_d(phi) / (60 h_d) with phi the inverse transform of P.  A layer on a
+// power-of-two mesh therefore transforms one mesh each way: k_grad6 turns the potential phi
 // into the forces F_d = -diff_d(phi) / (60 h_d), and k_div6 turns the
 // painted gradient meshes g_d into sum_d diff_d(g_d) / (60 h_d), whose
 // transform is the sum_d i D_d of theirs.
