@@ -2,7 +2,8 @@
 backward, against the FP64 layer on the same positions (FP32 values, cells of
 size one, so both see the same mesh coordinates): the fused pass at lengths on
 both sides of its launch shapes with partial strips, and the separate passes
-where the x axis is a power of two.  FP32 rounding is some 1e-6 of a norm here;
+where the x axis is a power of two; and power-of-two meshes on every route of
+the real-space stencils.  FP32 rounding is some 1e-6 of a norm here;
 1e-4 is what a single wrong column of the largest mesh exceeds many times."""
 import numpy as np
 import pytest
@@ -17,6 +18,8 @@ pytestmark = pytest.mark.gpu
 MESHES = [(5, 8, 6), (45, 20, 30), (100, 12, 18), (360, 24, 20), (500, 16, 12), (972, 6, 10), (1000, 5, 6), (12, 96, 180), (64, 30, 20), (128, 16, 48)]
 # columns enough for the shapes that fill the chip (more than 4096 in FP64, 8192 in FP32)
 MANY = [(20, 96, 180), (240, 96, 180), (360, 64, 270), (640, 48, 180), (810, 60, 150), (960, 64, 144), (1000, 48, 180)]
+# direct stencils up to 2^20 cells, marching ones 64, 256 and 128 (FP64 128) cells wide, partial tiles
+POW2 = [(4, 8, 8), (64, 16, 1024), (32, 64, 1024), (1024, 8, 256), (64, 256, 1024), (1024, 128, 128)]
 PRM = {"sm": [0.2, 0.7, 0.9, 4.0, 0.3], "dm": [0.2, 0.7, 0.9, 4.0, 0.3], "HI": [0.2, 0.7, 0.9, 4.0, 0.3, 0.1, 0.8, 1.1, 3.0, 0.2]}
 
 
@@ -41,6 +44,11 @@ def test_forces_and_adjoint_match_fp64(nm, kind):
 @pytest.mark.parametrize("nm", MANY, ids=str)
 def test_many_columns(nm, kind):
     compare(nm, kind)
+
+
+@pytest.mark.parametrize("nm", POW2, ids=str)
+def test_stencil_routes(nm):
+    compare(nm, "sm")
 
 
 def compare(nm, kind):
